@@ -54,7 +54,10 @@ namespace dopt {
 // (v_rcp_f32 and v_log_f32 each), and an element costs QMAX compares instead of an exp, a
 // reciprocal and the code arithmetic. The codes differ from the per-element form only for d within
 // the thresholds' fp32 error (about 1e-7) of a boundary; scale and min are computed as before.
-enum { PRE_NONE = 0, PRE_REF = 1, PRE_GELU = 2, PRE_SILU = 3 };
+//   PRE_SQ16  PRE_REF's squash (with or without the clamp) of bf16 inputs at 1 and 2 bits, nearest
+//             rounding: the same words, scale and min bit for bit, from thresholds on the bf16 grid
+//             (squash16_pass below); a wave it cannot serve takes PRE_REF's per-element code
+enum { PRE_NONE = 0, PRE_REF = 1, PRE_GELU = 2, PRE_SILU = 3, PRE_SQ16 = 4 };
 
 struct QuantPackArgs {
     const void* x;
@@ -170,6 +173,151 @@ __device__ __forceinline__ uint32_t pack_rne_codes(const float* z) {
     return acc;
 }
 
+// ------------------------------------------------------------------ squashed codes of bf16 inputs
+// bf16 bits <-> an int16 in the order of the values: negative values have their magnitude bits
+// inverted. -0 comes right below +0, NaNs above +inf (positive ones) and below -inf.
+typedef int16_t i16x2_t __attribute__((ext_vector_type(2)));
+constexpr int ORD_INF = 0x7f80, ORD_NEG_INF = -32641, ORD_NONE = 32767;
+
+__device__ __forceinline__ uint32_t order16x2(uint32_t w) {
+    const i16x2_t sign = __builtin_bit_cast(i16x2_t, w) >> 15;
+    return w ^ (__builtin_bit_cast(uint32_t, sign) & 0x7fff7fffu);
+}
+__device__ __forceinline__ float value16(int o) {
+    return __uint_as_float((uint32_t)(o ^ ((o >> 31) & 0x7fff)) << 16);
+}
+__device__ __forceinline__ i16x2_t as_i16x2(uint32_t w) { return __builtin_bit_cast(i16x2_t, w); }
+__device__ __forceinline__ uint32_t as_u32(i16x2_t v) { return __builtin_bit_cast(uint32_t, v); }
+
+// swap the bit fields of x selected by m with those d above them
+__device__ __forceinline__ uint32_t swap_fields(uint32_t x, int d, uint32_t m) {
+    const uint32_t t = (x ^ (x >> d)) & m;
+    return x ^ t ^ (t << d);
+}
+
+// PRE_SQ16: one lane's 16 * NP bf16 values of a group (NP pairs of 8-element units, raw words 8p..8p+7).
+//
+// The per-element form is code(x) = trunc(fma(squash(clamp(x)) - min, 1/step, 0.5 - 1e-6)), about 25
+// VALU instructions per element, two of them transcendental: on the ViT MLP activation (bf16
+// [128,197,3072], g = 512, 2-bit) the kernel was bound by them at 51.3 us (3.4 TB/s); it now takes 27.6 us
+// (6.3 TB/s; the nearest quantizer without the squash takes 25.3). Every part of it
+// is non-decreasing in x over the bf16 values (squash_half_tanh2 as evaluated here included: a test
+// walks all of them), so
+//   - min and max of the squashed values are the squash of the values' min and max, which are packed
+//     16-bit integer min / max of the ordered bits;
+//   - code >= k exactly when x >= b_k, the smallest bf16 value whose code is >= k. A lane finds its b_k
+//     from the inverse squash of the k-th rounding boundary, rounded to bf16, and the per-element form
+//     itself evaluated there and at the neighbour on the other side: two evaluations per lane instead of
+//     one per element. Lane j of a quad (a group spans whole quads) finds b_{j+1} and quad_perm
+//     broadcasts hand every lane all three.
+// An element then costs packed 16-bit saturating subtractions whose sign bits are its code.
+// A NaN in the wave, a neighbour pair that does not straddle the boundary (a boundary within the
+// inverse's error of zero, a saturated group) or an infinite 1/step sends the whole wave to the
+// per-element form: returns false and writes nothing.
+template <int BITS, int LPG, int NP>
+__device__ __forceinline__ bool squash16_pass(const QuantPackArgs& a, const uint32_t* raw, float& step, float& mn,
+                                              uint32_t* word) {
+    static_assert(BITS == 1 || BITS == 2, "threshold codes");
+    static_assert(LPG >= 4, "a group spans whole quads");
+    constexpr int QMAX = (1 << BITS) - 1;
+    const int lane = threadIdx.x & 63;
+    uint32_t o[8 * NP];
+#pragma unroll
+    for (int j = 0; j < 8 * NP; ++j) o[j] = order16x2(raw[j]);
+    i16x2_t lo = as_i16x2(o[0]), hi = as_i16x2(o[0]);
+#pragma unroll
+    for (int j = 1; j < 8 * NP; ++j) {
+        lo = __builtin_elementwise_min(lo, as_i16x2(o[j]));
+        hi = __builtin_elementwise_max(hi, as_i16x2(o[j]));
+    }
+    const int lo_i = min((int)lo.x, (int)lo.y), hi_i = max((int)hi.x, (int)hi.y);
+    const bool nan = lo_i < ORD_NEG_INF || hi_i > ORD_INF;
+    float xmn = value16(lo_i), xmx = value16(hi_i);
+    group_minmax<LPG>(xmn, xmx);
+
+    const bool clamp = a.flags & FL_CLAMP;
+    const float al = a.clamp_alpha, half_m = 0.49999899f;  // fp32(0.5 - 1e-6)
+    auto squash = [&](float x) { return squash_half_tanh2(clamp ? __builtin_amdgcn_fmed3f(x, -al, al) : x); };
+    // even lanes squash the group's min, odd lanes its max (a group holds whole lane pairs)
+    const float own = squash((lane & 1) ? xmx : xmn), other = dpp_f32<0xB1>(own);
+    mn = ((lane & 1) ? other : own) + 0.0f;  // store -0.0 as +0.0
+    const float rng = ((lane & 1) ? own : other) - mn;
+    step = rng > 0.0f ? div_by_qmax<QMAX>(rng) : 1.0f;
+    const float inv = exact_rcp(step);
+
+    // this lane's boundary. First y, the smallest float with fma(y, 1/step, 0.5 - 1e-6) >= k, among the
+    // eight around (k - (0.5 - 1e-6)) step; then s, from which on squash - min rounds to y or more (half a
+    // spacing below min + y: on data symmetric about zero a boundary lies as close to zero as the
+    // rounding of squash - min, where bf16 is finer than that); then x = atanh(2s) / 2 (a series below
+    // |s| = 0.1, where the logarithm's absolute error would exceed the bf16 spacing of x)
+    const int k = QMAX == 1 ? 1 : ((lane & 3) < 2 ? (lane & 3) + 1 : 3);
+    const float kf = (float)k;
+    uint32_t yb = __float_as_uint((kf - half_m) * step) - 4u;
+#pragma unroll
+    for (uint32_t w = 4; w; w >>= 1)
+        yb += __builtin_fmaf(__uint_as_float(yb + w - 1u), inv, half_m) >= kf ? 0u : w;
+    const float y = __uint_as_float(yb);
+    const float s = (y + mn) - 0.5f * (y - __uint_as_float(yb - 1u)), s2 = s * s;
+    const float series = s * __builtin_fmaf(s2, __builtin_fmaf(s2, __builtin_fmaf(s2, 64.0f / 7.0f, 3.2f), 4.0f / 3.0f), 1.0f);
+    const float logit = 0.17328679513998632f * __builtin_amdgcn_logf((0.5f + s) * __builtin_amdgcn_rcpf(0.5f - s));
+    const float t = fabsf(s) < 0.1f ? series : logit;
+    const uint32_t tb = to_bf16(t);
+    const int c = (int)(int16_t)(uint16_t)(tb ^ ((tb & 0x8000u) ? 0x7fffu : 0u));
+    auto reached = [&](int ord) {
+        return (int)cvt_u32(__builtin_fmaf(squash(value16(ord)) - mn, inv, half_m)) >= k;
+    };
+    const bool at = reached(c);
+    const bool beside = reached(at ? c - 1 : c + 1);
+    const bool constant = !(rng > 0.0f);  // every code is 0
+    if (wave_any(nan || inv == __builtin_inff() || (at == beside && !constant))) return false;
+    const int b = constant ? ORD_NONE : (at ? c : c + 1);
+    const uint32_t u = ((uint32_t)(b - 1) & 0xffffu) * 0x10001u;  // b - 1 in both halves: o > u is o >= b
+
+    const i16x2_t u1 = as_i16x2(dpp_u32<0x00>(u)), u2 = as_i16x2(dpp_u32<0x55>(u)), u3 = as_i16x2(dpp_u32<0xAA>(u));
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+        uint32_t acc[2] = {0u, 0u};
+        if constexpr (BITS == 2) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const i16x2_t e = as_i16x2(o[8 * p + j]);
+                const uint32_t d1 = as_u32(__builtin_elementwise_sub_sat(u1, e));
+                const uint32_t d2 = as_u32(__builtin_elementwise_sub_sat(u2, e));
+                const uint32_t d3 = as_u32(__builtin_elementwise_sub_sat(u3, e));
+                const uint32_t low = (d1 & ~d2) | d3;  // sign bits: the code's low bit; d2's are its high bit
+                const uint32_t two = (d2 & 0x80008000u) | ((low >> 1) & ~0x80008000u);
+                acc[j >> 2] = (acc[j >> 2] >> 2) | (two & 0xC000C000u);
+            }
+            // byte 1 of acc: the unit's four even elements' codes, byte 3: its odd elements'
+            uint32_t w = __builtin_amdgcn_perm(acc[1], acc[0], 0x07050301u);
+            w = swap_fields(w, 4, 0x00F000F0u);
+            w = swap_fields(w, 2, 0x0C0C0C0Cu);
+            // the low half holds the first unit's codes, the high half the second's: even lanes take the
+            // lane pair's first-unit dword, odd lanes its second-unit dword
+            const uint32_t n = dpp_u32<0xB1>(w);
+            word[p] = __builtin_amdgcn_perm(n, w, (lane & 1) ? 0x03020706u : 0x05040100u);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                acc[j >> 2] = (acc[j >> 2] >> 1) |
+                              (as_u32(__builtin_elementwise_sub_sat(u1, as_i16x2(o[8 * p + j]))) & 0x80008000u);
+            // bits 15:12 of acc: the even elements' codes, bits 31:28 the odd elements'
+            const uint32_t both = (acc[1] & 0xF000F000u) | ((acc[0] >> 4) & 0x0F000F00u);
+            uint32_t w = __builtin_amdgcn_perm(0u, both, 0x0C0C0301u);
+            w = swap_fields(w, 4, 0x00F0u);
+            w = swap_fields(w, 2, 0x0C0Cu);
+            w = swap_fields(w, 1, 0x2222u);
+            // byte 0: the first unit's codes, byte 1: the second's; lane 0 of a quad takes the quad's
+            // first-unit dword, lane 1 its second-unit dword
+            const uint32_t n1 = dpp_u32<0xB1>(w);
+            const uint32_t z = __builtin_amdgcn_perm(n1, w, (lane & 1) ? 0x01050004u : 0x05010400u);
+            const uint32_t n2 = dpp_u32<0x4E>(z);
+            word[p] = __builtin_amdgcn_perm(n2, z, (lane & 1) ? 0x07060302u : 0x05040100u);
+        }
+    }
+    return true;
+}
+
 template <int DT, int BITS, int G, int RN, int UB, int LPG_, int P, int PRE, bool NT, bool TILED>
 __global__ __launch_bounds__(256) void quant_pack_kernel(QuantPackArgs a) {
     using C = QuantPackCfg<DT, BITS, G, RN, UB, LPG_, P>;
@@ -220,12 +368,32 @@ __global__ __launch_bounds__(256) void quant_pack_kernel(QuantPackArgs a) {
     #pragma unroll
     for (int p = 0; p < P; ++p) {
         const uint32_t r = g0 + p * GPP + slot;
+        if constexpr (PRE == PRE_SQ16) {
+            static_assert(DT == DT_BF16 && RN == RN_NEAREST && P == 1 && CPL % 2 == 0 && UE == 8, "squash16_pass's lane");
+            uint32_t w[4 * CPL], word[CPL / 2];
+#pragma unroll
+            for (int i = 0; i < CPL; ++i) {
+                w[4 * i] = raw[p][i][0].x;
+                w[4 * i + 1] = raw[p][i][0].y;
+                w[4 * i + 2] = raw[p][i][0].z;
+                w[4 * i + 3] = raw[p][i][0].w;
+            }
+            if (squash16_pass<BITS, LPG, CPL / 2>(a, w, step_p[p], mn_p[p], word)) {
+                constexpr int LPD = 32 / UBITS;  // lanes whose units share a dword
+                const int unit = li % LPD;       // 0: the lane holds its pair's / quad's first-unit dword, 1: the second's
+                uint32_t* dst = a.packed + (uint64_t)r * W + li / LPD + unit * (LPG / LPD);
+#pragma unroll
+                for (int q = 0; q < CPL / 2; ++q)
+                    if (r < a.n_groups && unit < 2) dst[q * (2 * LPG / LPD)] = word[q];
+                continue;
+            }
+        }
         float v[CPL][UE];
         #pragma unroll
         for (int i = 0; i < CPL; ++i)
             #pragma unroll
             for (int l = 0; l < LOADS; ++l) widen16<DT>(raw[p][i][l], &v[i][l * E16]);
-        if constexpr (PRE == PRE_REF) {
+        if constexpr (PRE == PRE_REF || PRE == PRE_SQ16) {
             if (a.flags & FL_CLAMP) {
                 // one v_med3 per element equals fminf(fmaxf(x, -alpha), alpha) for alpha >= 0,
                 // NaN x included (med3 of a NaN and two numbers is their minimum, here -alpha)

@@ -26,8 +26,11 @@ struct QuantPackShape {
     // 3% faster than two units per lane on bf16 [256,256,56,56], g = 256, 2-bit); otherwise two. The fused activations run
     // GELU with two passes per wave, SiLU with one: measured on the ViT MLP activation (bf16
     // [256,197,3072], g = 128) over 1-16 units per lane and 1-4 passes, two units per lane gave
-    // the fastest kernels at 1-8 bits (four units, 108 VGPRs for GELU, ran 4-10% slower)
-    static constexpr int L0 = RN == RN_NOISE || RN == RN_PHILOX ? CPG : CPG / 2;
+    // the fastest kernels at 1-8 bits (four units, 108 VGPRs for GELU, ran 4-10% slower). The squashed
+    // bf16 quantizer finds its thresholds once per lane, about 130 instructions, so a lane takes eight
+    // units (never fewer than four lanes per group): bf16 [128,197,3072], g = 512, 2-bit, 42.0 / 29.9 /
+    // 27.6 us with two / four / eight units (51.3 us in the per-element form)
+    static constexpr int L0 = RN == RN_NOISE || RN == RN_PHILOX ? CPG : PRE == PRE_SQ16 ? (CPG < 32 ? 4 : CPG / 8) : CPG / 2;
     static constexpr int L1 = L0 < LPD ? LPD : L0;
     static constexpr int L2 = L1 < 2 ? 2 : L1;
     static constexpr int LPG = L2 > 64 ? 64 : L2;
@@ -58,7 +61,15 @@ template <int DT, int BITS, int G>
 static int qp_rn(const QuantPackArgs& a, int rn, int pre, hipStream_t s) {
     if (pre == PRE_REF) {  // the reference quantizer's clamp / squash, with any rounding
         switch (rn) {
-            case RN_NEAREST: return qp_launch<DT, BITS, G, RN_NEAREST, PRE_REF>(a, s);
+            case RN_NEAREST:
+                // threshold codes on the bf16 grid where the squash applies (4 and 8 bits would need 15 and
+                // 255 thresholds; an fp32 or fp16 input has no grid on which the evaluated squash was shown
+                // non-decreasing); a negative or NaN alpha keeps the per-element clamp's own arithmetic
+                if constexpr (DT == DT_BF16 && BITS <= 2) {
+                    if ((a.flags & FL_SQUASH) && (!(a.flags & FL_CLAMP) || a.clamp_alpha >= 0.0f))
+                        return qp_launch<DT, BITS, G, RN_NEAREST, PRE_SQ16>(a, s);
+                }
+                return qp_launch<DT, BITS, G, RN_NEAREST, PRE_REF>(a, s);
             case RN_NOISE: return qp_launch<DT, BITS, G, RN_NOISE, PRE_REF>(a, s);
             case RN_PHILOX: return qp_launch<DT, BITS, G, RN_PHILOX, PRE_REF>(a, s);
         }
