@@ -1,12 +1,16 @@
-// FP8 e4m3 scaled GEMM launcher (kernels and tiling in fp8_gemm.h).
+// FP8 e4m3 scaled GEMM launcher: which kernel and tile a shape gets.
 //
-// Configuration: 256 x 256 workgroup tiles (128 x 128 per wave), GROUP_M = 4 tile rows per
-// L2 group, even MFMA / memory interleave; the persistent kernels with one workgroup per CU
-// (16x16x128 MFMAs from K = 8192, 32x32x64 below; the non-persistent kernel for an odd number of
-// K slabs); measured on MI355X at 8192^3 and 4096x11008x4096.
+// Large outputs take 256 x 256 tiles (fp8_gemm.h: GROUP_M = 4 tile rows per L2 group, even MFMA / memory
+// interleave; the persistent kernels with one workgroup per CU, 16x16x128 MFMAs from K = 8192, 32x32x64
+// below; the non-persistent kernel for an odd number of K slabs). They leave CUs idle when the output has
+// few of them, and a tile's K slabs run one after the other: M = 64, N = K = 4096 took 38 us on 16
+// workgroups. Smaller outputs take smaller tiles (fp8_gemm_mid.h, fp8_gemm_small.h) by the estimate in
+// `plan` below.
 #include <atomic>
 
 #include "fp8_gemm.h"
+#include "fp8_gemm_mid.h"
+#include "fp8_gemm_small.h"
 
 namespace dopt {
 
@@ -28,10 +32,69 @@ int device_cu_count() {
 }
 }  // namespace
 
+namespace {
+
+using Fp8Gemm128 = Fp8GemmCfg<128, 128, 4, 0>;
+
+// Estimated time (us) of a tile shape on this part: start + per K slab the larger of a lone workgroup's
+// step and the CU's throughput at its share of the tiles, + an epilogue per round of tiles. The constants
+// are fitted to a sweep in which every kernel was timed on 32 shapes from 1 x 4096 x 4096 to 4096^3; on
+// those the estimate picks the fastest kernel or one within 10% of it but for rows that are not a
+// multiple of 128 bytes (within 25%). Times in us, before (256 x 256 tiles only) -> now: 16 x 768 x 768
+// 12.1 -> 3.0, 64 x 4096 x 4096 38 -> 7.2, 256 x 256 x 8192 64 -> 8.3, 985 x 3072 x 768 15.0 -> 7.1,
+// 1024^3 13.3 -> 4.2, 1024 x 4096 x 4096 38 -> 19.1, 2048^3 21.8 -> 12.0; from about 3000^3 on the
+// 256 x 256 tiles are the fastest and stay.
+struct TileCost {
+    int bm, bn;
+    float start, step, rate, epilogue;
+};
+enum { T_SMALL, T_32x64, T_64x64, T_128x64, T_128x128, T_128x128_NT, T_256, T_COUNT };
+constexpr TileCost TILE_COST[T_COUNT] = {
+    {16, 16, 2.4f, 0.09f, 0.105f, 0.1f},   // 8 waves split K (M <= 16 only)
+    {32, 64, 2.2f, 0.14f, 0.14f, 0.4f},
+    {64, 64, 2.4f, 0.17f, 0.18f, 0.8f},
+    {128, 64, 2.9f, 0.20f, 0.29f, 1.2f},
+    {128, 128, 2.9f, 0.33f, 0.50f, 1.8f},
+    {128, 128, 2.9f, 0.60f, 0.50f, 1.5f},  // two workgroups per CU, double-buffered (hides part of its epilogues)
+    {256, 256, 5.0f, 0.95f, 1.45f, 2.5f},
+};
+
+int plan(int64_t M, int64_t N, int64_t K, int n_cu) {
+    const float nk = (float)((K + 127) / 128);
+    int best = T_256;
+    float least = 0.0f;
+    for (int t = T_COUNT - 1; t >= 0; --t) {
+        const TileCost& c = TILE_COST[t];
+        if (t == T_SMALL && M > 16) continue;
+        const int64_t tiles = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
+        if (tiles >= ((int64_t)1 << 31)) continue;
+        const float rounds = (float)((tiles + n_cu - 1) / n_cu);
+        const float step = c.rate * rounds > c.step ? c.rate * rounds : c.step;
+        const float us = c.start + nk * step + c.epilogue * rounds;
+        if (t == T_256 || us < least) {
+            least = us;
+            best = t;
+        }
+    }
+    return best;
+}
+
+}  // namespace
+
 int launch_fp8_gemm_nt(const uint8_t* A, const uint8_t* B, int64_t M, int64_t N, int64_t K, int64_t lda,
                        int64_t ldb, float out_scale, uint16_t* C, int64_t ldc, hipStream_t s) {
-    return fp8_gemm_persistent_launch<Fp8GemmDefault>(A, B, M, N, K, lda, ldb, out_scale, C, ldc,
-                                                      device_cu_count(), s);
+    const int n_cu = device_cu_count();
+    const Fp8GemmArgs p{A, B, C, M, N, K, lda, ldb, ldc, out_scale, 0, 0,
+                        (uint32_t)(ldc % 8 == 0 && ((uintptr_t)C & 15) == 0)};
+    switch (plan(M, N, K, n_cu)) {
+        case T_SMALL: return fp8_gemm_small_launch<1, 1, 8>(p, s);
+        case T_32x64: return fp8_gemm_mid_launch<32, 64>(p, s);
+        case T_64x64: return fp8_gemm_mid_launch<64, 64>(p, s);
+        case T_128x64: return fp8_gemm_mid_launch<128, 64>(p, s);
+        case T_128x128: return fp8_gemm_mid_launch<128, 128>(p, s);
+        case T_128x128_NT: return fp8_gemm_launch<Fp8Gemm128>(A, B, M, N, K, lda, ldb, out_scale, C, ldc, s);
+    }
+    return fp8_gemm_persistent_launch<Fp8GemmDefault>(A, B, M, N, K, lda, ldb, out_scale, C, ldc, n_cu, s);
 }
 
 }  // namespace dopt
