@@ -6,57 +6,109 @@
 // and B [K, N] with arbitrary strides, so B in its natural row-major [K, N] layout (stride_r =
 // 1 along N, stride_c = ldb along K) is transposed here into [N, K].
 //
-// Two kernels:
-//   - transpose (stride_r == 1): 64 x 64 byte tiles through LDS; each lane reads 16 contiguous
-//     source bytes (one column c, rows r..r+15) and, after the LDS round trip, writes 16
-//     contiguous destination bytes (one row r, columns c..c+15). The LDS tile is padded by 16
-//     bytes per row so the column-wise writes fall in different banks.
+// Three kernels:
+//   - transpose (stride_r == 1): 128 x 128 byte tiles. A lane reads 16 contiguous source bytes (rows
+//     r..r+15) of four columns c..c+3, transposes the sixteen 4-byte rows in registers (v_perm_b32) and
+//     writes them to LDS as dwords; after the barrier it writes 16 contiguous destination bytes of one row
+//     per step. Rows of the LDS tile are 33 dwords apart, so the dword writes of 8 lanes 16 rows apart fall
+//     in different banks. Bound by HBM: [8192, 8192] takes 20.8 us, 6.4 TB/s, and 42.7 us on [8191, 8191],
+//     whose unaligned lines are read twice (64 x 64 tiles moved byte by byte: 31.1 and 101 us).
+//   - copy (stride_c == 1): whole rows whose pitch or base does not suit the GEMM; 16 bytes per lane
+//     ([8192, 8192] 20.2 us; 93.6 us through the gather).
 //   - gather (anything else): one byte per lane, consecutive lanes along c.
+// Source addresses need no alignment: 16-byte loads from any byte are one instruction on gfx950.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 namespace dopt {
 
-constexpr int TP = 64;  // tile edge (bytes)
+constexpr int TP = 128;          // tile edge (bytes)
+constexpr int TPITCH = TP / 4 + 1;  // dwords per LDS row
+
+// 16 bytes from any address
+__device__ __forceinline__ uint4 load16_any(const uint8_t* p) {
+    uint4 v;
+    __builtin_memcpy(&v, p, 16);
+    return v;
+}
 
 __global__ __launch_bounds__(256) void fp8_transpose_kernel(const uint8_t* __restrict__ src, int64_t rows,
                                                             int64_t cols, int64_t stride_c, uint8_t* __restrict__ dst,
                                                             int64_t ld_dst, uint32_t row_tiles) {
-    __shared__ uint8_t t[TP][TP + 16];
+    __shared__ uint32_t t[TP * TPITCH];
     const int64_t r0 = (int64_t)(blockIdx.x % row_tiles) * TP, c0 = (int64_t)(blockIdx.x / row_tiles) * TP;
-    const int lane = threadIdx.x;
-    // read: lane -> column c0 + lane / 4, rows r0 + 16 (lane % 4) .. +15 (contiguous in src)
+    const int tid = threadIdx.x;
     {
-        const int cl = lane >> 2, rl = (lane & 3) * 16;
-        const int64_t c = c0 + cl, r = r0 + rl;
-        uint8_t v[16];
-        if (c < cols && r + 16 <= rows && (((uintptr_t)(src + c * stride_c + r)) & 15) == 0) {
-            const uint4 x = *(const uint4*)(src + c * stride_c + r);
-            const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+        const int rl = (tid & 7) * 16, cl = (tid >> 3) * 4;  // this lane's 16 x 4 block
+        const int64_t r = r0 + rl;
+        uint32_t w[4][4];  // [column][dword of its 16 rows]
 #pragma unroll
-            for (int i = 0; i < 16; ++i) v[i] = (uint8_t)(w[i >> 2] >> (8 * (i & 3)));
-        } else {
+        for (int j = 0; j < 4; ++j) {
+            const int64_t c = c0 + cl + j;
+            if (c < cols && r + 16 <= rows) {
+                const uint4 v = load16_any(src + c * stride_c + r);
+                w[j][0] = v.x;
+                w[j][1] = v.y;
+                w[j][2] = v.z;
+                w[j][3] = v.w;
+            } else {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) v[i] = (c < cols && r + i < rows) ? src[c * stride_c + r + i] : 0;
+                for (int q = 0; q < 4; ++q) {
+                    w[j][q] = 0;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (c < cols && r + 4 * q + e < rows) w[j][q] |= (uint32_t)src[c * stride_c + r + 4 * q + e] << (8 * e);
+                }
+            }
         }
 #pragma unroll
-        for (int i = 0; i < 16; ++i) t[rl + i][cl] = v[i];
+        for (int q = 0; q < 4; ++q) {
+            // a 4 x 4 byte block: rows 4q..4q+3 of the four columns
+            const uint32_t lo01 = __builtin_amdgcn_perm(w[1][q], w[0][q], 0x05010400u);  // a0 b0 a1 b1
+            const uint32_t hi01 = __builtin_amdgcn_perm(w[1][q], w[0][q], 0x07030602u);  // a2 b2 a3 b3
+            const uint32_t lo23 = __builtin_amdgcn_perm(w[3][q], w[2][q], 0x05010400u);
+            const uint32_t hi23 = __builtin_amdgcn_perm(w[3][q], w[2][q], 0x07030602u);
+            uint32_t* at = t + (rl + 4 * q) * TPITCH + (cl >> 2);
+            at[0] = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u);
+            at[TPITCH] = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u);
+            at[2 * TPITCH] = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
+            at[3 * TPITCH] = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
+        }
     }
     __syncthreads();
-    // write: lane -> row r0 + lane / 4, columns c0 + 16 (lane % 4) .. +15 (contiguous in dst)
-    {
-        const int rl = lane >> 2, cl = (lane & 3) * 16;
-        const int64_t r = r0 + rl, c = c0 + cl;
-        if (r >= rows) return;
+    const int cl = (tid & 7) * 16;
+    const int64_t c = c0 + cl;
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+        const int rl = (tid >> 3) + 32 * h;
+        const int64_t r = r0 + rl;
+        if (r >= rows || c >= cols) continue;
+        const uint32_t* s = t + rl * TPITCH + (cl >> 2);
+        const uint32_t v[4] = {s[0], s[1], s[2], s[3]};
         uint8_t* d = dst + r * ld_dst + c;
         if (c + 16 <= cols && (((uintptr_t)d) & 15) == 0) {
-            uint32_t w[4] = {0, 0, 0, 0};
-#pragma unroll
-            for (int i = 0; i < 16; ++i) w[i >> 2] |= (uint32_t)t[rl][cl + i] << (8 * (i & 3));
-            *(uint4*)d = make_uint4(w[0], w[1], w[2], w[3]);
+            *(uint4*)d = make_uint4(v[0], v[1], v[2], v[3]);
         } else {
-            for (int i = 0; i < 16 && c + i < cols; ++i) d[i] = t[rl][cl + i];
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                if (c + i < cols) d[i] = (uint8_t)(v[i >> 2] >> (8 * (i & 3)));
         }
+    }
+}
+
+// rows of `cols` contiguous bytes: lane -> 16 bytes of one row
+__global__ __launch_bounds__(256) void fp8_copy_rows_kernel(const uint8_t* __restrict__ src, int64_t cols,
+                                                            int64_t stride_r, uint8_t* __restrict__ dst, int64_t ld_dst,
+                                                            uint64_t chunks, uint32_t per_row) {
+    const uint64_t q = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    if (q >= chunks) return;
+    const int64_t r = (int64_t)(q / per_row), c = (int64_t)(q % per_row) * 16;
+    const uint8_t* s = src + r * stride_r + c;
+    uint8_t* d = dst + r * ld_dst + c;
+    if (c + 16 <= cols && (((uintptr_t)d) & 15) == 0) {
+        *(uint4*)d = load16_any(s);
+    } else {
+        for (int i = 0; i < 16 && c + i < cols; ++i) d[i] = s[i];
     }
 }
 
@@ -76,6 +128,11 @@ int launch_fp8_pack(const uint8_t* src, int64_t rows, int64_t cols, int64_t stri
         if (rt * ct >= (1ull << 31)) return -1;
         hipLaunchKernelGGL(fp8_transpose_kernel, dim3((uint32_t)(rt * ct)), dim3(256), 0, s, src, rows, cols, stride_c,
                            dst, ld_dst, (uint32_t)rt);
+    } else if (stride_c == 1) {
+        const uint64_t pr = (uint64_t)((cols + 15) / 16), chunks = (uint64_t)rows * pr;
+        if (pr >= (1ull << 32) || (chunks + 255) / 256 >= (1ull << 31)) return -1;
+        hipLaunchKernelGGL(fp8_copy_rows_kernel, dim3((uint32_t)((chunks + 255) / 256)), dim3(256), 0, s, src, cols,
+                           stride_r, dst, ld_dst, chunks, (uint32_t)pr);
     } else {
         const uint64_t cb = (uint64_t)((cols + 255) / 256);
         if ((uint64_t)rows * cb >= (1ull << 31)) return -1;
