@@ -50,6 +50,8 @@ EXPORTS = (
     "dopt_bn_bwd_dx_alam",
     "dopt_dw_gemm_workspace_floats",
     "dopt_dw_gemm",
+    "dopt_dw_gemm_any_workspace_floats",
+    "dopt_dw_gemm_any",
     "dopt_graph_node_counts",
     "dopt_graph_replace_memsets",
     "dopt_alam_quant_pack",
@@ -153,6 +155,10 @@ def lib() -> ctypes.CDLL:
         L.dopt_dw_gemm_workspace_floats.restype = i64
         L.dopt_dw_gemm.argtypes = [vp, i64, vp, i64, vp, vp, vp, i32, i32, i64, i64, i64, vp, vp, vp, vp, vp]
         L.dopt_dw_gemm.restype = i32
+        L.dopt_dw_gemm_any_workspace_floats.argtypes = [i64, i64, i64]
+        L.dopt_dw_gemm_any_workspace_floats.restype = i64
+        L.dopt_dw_gemm_any.argtypes = [vp, i64, vp, i64, i64, i64, i64, vp, vp, vp, vp, vp]
+        L.dopt_dw_gemm_any.restype = i32
         L.dopt_graph_node_counts.argtypes = [vp, vp, i32]
         L.dopt_graph_node_counts.restype = i32
         L.dopt_graph_replace_memsets.argtypes = [vp, vp]

@@ -956,6 +956,43 @@ int dopt_dw_gemm(const void* dy, int64_t ldd, const void* x_hat, int64_t ldx, co
 
 }  // extern "C"
 
+static bool dw_any_shape(int64_t M, int64_t N, int64_t K) {
+    return M > 0 && N > 0 && K >= 0 && M % 8 == 0 && N % 8 == 0 && M < ((int64_t)1 << 20) && N < ((int64_t)1 << 20) &&
+           K < ((int64_t)1 << 31);
+}
+
+int64_t dopt_dw_gemm_any_workspace_floats(int64_t M, int64_t N, int64_t K) {
+    return dw_any_shape(M, N, K) ? dopt::dw_workspace_floats(M, N, K) : 0;
+}
+
+int dopt_dw_gemm_any(const void* dy, int64_t ldd, const void* x_hat, int64_t ldx, int64_t M, int64_t N, int64_t K,
+                     float* workspace, float* dw_f32, void* dw_bf16, float* db, void* stream) {
+    if (!dw_any_shape(M, N, K))
+        return fail(DOPT_EUNSUPPORTED, "dw_gemm_any needs M and N positive multiples of 8 below 2^20 (got M=%lld N=%lld K=%lld)",
+                    (long long)M, (long long)N, (long long)K);
+    if ((K > 0 && (!dy || !x_hat)) || !workspace || (!dw_f32 && !dw_bf16))
+        return fail(DOPT_EINVAL, "null dy/x_hat/workspace/output pointer");
+    if (ldd < M || ldd % 8 || ldd >= ((int64_t)1 << 24) || !aligned16(dy) || ldx < N || ldx % 8 ||
+        ldx >= ((int64_t)1 << 24) || !aligned16(x_hat))
+        return fail(DOPT_EINVAL, "dy and x_hat must be 16-byte aligned, their row strides multiples of 8, at least M and N "
+                                 "and below 2^24");
+    if (((uintptr_t)workspace & 15u) || (dw_f32 && ((uintptr_t)dw_f32 & 15u)) || (dw_bf16 && ((uintptr_t)dw_bf16 & 7u)))
+        return fail(DOPT_EINVAL, "workspace / dw_f32 must be 16-byte and dw_bf16 8-byte aligned");
+    dopt::DwArgs a{};
+    a.dy = (const uint16_t*)dy;
+    a.ldd = ldd;
+    a.xh = (const uint16_t*)x_hat;
+    a.ldx = ldx;
+    a.M = M;
+    a.N = N;
+    a.K = K;
+    a.partial = workspace;
+    (void)hipGetLastError();
+    if (dopt::launch_dw_gemm(a, dopt::DW_B_BF16, db != nullptr, dw_f32, (uint16_t*)dw_bf16, db, (hipStream_t)stream))
+        return fail(DOPT_EUNSUPPORTED, "no dw_gemm_any kernel for this shape");
+    return hip_status("dw_gemm_any launch");
+}
+
 int dopt_graph_node_counts(void* graph, int64_t* counts, int n_counts) {
     if (!graph || (!counts && n_counts > 0) || n_counts < 0) return fail(DOPT_EINVAL, "null graph or counts");
     for (int i = 0; i < n_counts; ++i) counts[i] = 0;

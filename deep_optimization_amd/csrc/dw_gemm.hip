@@ -28,6 +28,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <cmath>
 
 #include "dopt_device.h"
 #include "dw_gemm.h"
@@ -260,8 +261,8 @@ __global__ __launch_bounds__(THREADS, 1) void dw_gemm_kernel(DwArgs a) {
 // LDS rows are 512 bytes (256 bf16); 16-byte chunk c of row r sits at position c ^ (4 * (r % 4)),
 // which puts the 4 rows of a transposing read on 4 distinct 64-byte bank groups.
 constexpr int V2_BK = 32;
+constexpr uint32_t BUF_OOB = 0x80000000u;  // or'ed into an offset: past any buffer resource's range
 constexpr int V2_ROWB = 512;                    // bytes per LDS row (256 bf16)
-constexpr int V2_TILE = V2_BK * V2_ROWB;        // bytes of one operand tile (16 KB)
 
 typedef short v4i16_t __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
@@ -348,15 +349,28 @@ struct V2Codes {
 // workgroup tile, the DMA ring and the order of the MFMA steps are the same either way.
 // BMT: output rows per workgroup tile, 256 or (for small outputs, so fewer K splits fill the GPU
 // and fewer split partials go through HBM) 128; the waves then cover 64 rows each.
-template <int BITS, bool DB, int NW, int BMT>
+//
+// RAG (bf16 x_hat): any K, M and N multiples of 8. The tiles arrive through buffer resources whose record
+// count ends at row K of the slab (rows past it read zeros, so a short last slab adds nothing), lanes whose
+// 8 columns lie past M (N) load beyond the range, and the partial tile's stores are masked. The main loop
+// is the same: 3072 x 768 over 25216 tokens runs in the same time through either instance (128 us). A K that
+// is no multiple of 32 had gone through dw_gemm_kernel (768 x 3072 over 3645 tokens 51 -> 40 us), and other M, N
+// through torch's product and sum (384 x 1536 over 6304 tokens 68 -> 25 us, 640 x 640 over 12000 100 -> 23 us).
+// BNT: output columns per workgroup tile (256, or 128 for RAG).
+template <int BITS, bool DB, int NW, int BMT, int BNT = 256, bool RAG = false>
 __global__ __launch_bounds__(64 * NW, 1) void dw_gemm_v2_kernel(DwArgs a) {
     static_assert(BITS == 0 || BITS == 1 || BITS == 2 || BITS == 4, "bf16, or 1/2/4-bit codes");
     static_assert(NW == 4 || (NW == 8 && BITS == 0), "8 waves for bf16 x_hat only");
+    static_assert(BNT == 256 || (BNT == 128 && RAG), "narrow x_hat tiles for the ragged kernel only");
+    static_assert(!RAG || BITS == 0, "ragged shapes: bf16 x_hat only");
     using CS = V2Codes<BITS>;
     constexpr int WN = NW / 2;            // waves along n
-    constexpr int CW = BN / WN;           // columns per wave
+    constexpr int CW = BNT / WN;          // columns per wave
     constexpr int TNW = CW / 32;          // 32 x 32 blocks per wave along n
-    constexpr int JJ = 16 / NW;           // 1 KB DMA blocks per wave per x_hat tile
+    constexpr int RB = BNT * 2;           // bytes per LDS row of an x_hat tile
+    constexpr int TILE_B = V2_BK * RB;    // bytes of one x_hat tile
+    constexpr int JJ = TILE_B / 1024 / NW;  // 1 KB DMA blocks per wave per x_hat tile
+    constexpr int RPBB = 1024 / RB, LPRB = RB / 16;  // x_hat rows per block, lanes per row
     static_assert(BMT == 256 || BMT == 128, "tile rows");
     constexpr int RA = BMT * 2;           // bytes per LDS row of a dy tile
     constexpr int TILE_A = V2_BK * RA;    // bytes of one dy tile
@@ -370,16 +384,16 @@ __global__ __launch_bounds__(64 * NW, 1) void dw_gemm_v2_kernel(DwArgs a) {
     __shared__ __attribute__((aligned(1024))) char sa1[TILE_A];
     __shared__ __attribute__((aligned(1024))) char sa2[TILE_A];
     __shared__ __attribute__((aligned(1024))) char sa3[TILE_A];
-    __shared__ __attribute__((aligned(1024))) char sb0[V2_TILE];
-    __shared__ __attribute__((aligned(1024))) char sb1[V2_TILE];
-    __shared__ __attribute__((aligned(1024))) char sb2[V2_TILE];
-    __shared__ __attribute__((aligned(1024))) char sb3[V2_TILE];
+    __shared__ __attribute__((aligned(1024))) char sb0[TILE_B];
+    __shared__ __attribute__((aligned(1024))) char sb1[TILE_B];
+    __shared__ __attribute__((aligned(1024))) char sb2[TILE_B];
+    __shared__ __attribute__((aligned(1024))) char sb3[TILE_B];
     __shared__ __attribute__((aligned(1024))) char sc0[CS::SLOT];
     __shared__ __attribute__((aligned(1024))) char sc1[CS::SLOT];
     __shared__ __attribute__((aligned(1024))) char sc2[CS::SLOT];
     __shared__ __attribute__((aligned(1024))) char sc3[CS::SLOT];
 
-    const int tiles_n = (int)(a.N / BN), tiles = (int)(a.M / BMT) * tiles_n;
+    const int tiles_n = (int)((a.N + BNT - 1) / BNT), tiles = (int)((a.M + BMT - 1) / BMT) * tiles_n;
     const int W = tiles * a.splits, per = (W + DW_XCDS - 1) / DW_XCDS;
     const int xcd = blockIdx.x % DW_XCDS, local = blockIdx.x / DW_XCDS;
     if (local >= per) return;
@@ -387,9 +401,9 @@ __global__ __launch_bounds__(64 * NW, 1) void dw_gemm_v2_kernel(DwArgs a) {
     if (L >= W) return;
     const int split = L / tiles, t = L % tiles;
     const int tm = t / tiles_n, tn = t % tiles_n;
-    const int64_t m0 = (int64_t)tm * BMT, n0 = (int64_t)tn * BN;
+    const int64_t m0 = (int64_t)tm * BMT, n0 = (int64_t)tn * BNT;
     const int64_t kt0 = (int64_t)split * a.kt_per_split;
-    const int64_t kt1 = min(kt0 + a.kt_per_split, a.K / V2_BK);
+    const int64_t kt1 = min(kt0 + a.kt_per_split, (a.K + V2_BK - 1) / V2_BK);
     const int nk = (int)(kt1 - kt0);
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -409,11 +423,13 @@ __global__ __launch_bounds__(64 * NW, 1) void dw_gemm_v2_kernel(DwArgs a) {
     for (int j = 0; j < JA; ++j) {
         const int r = RPB * (NW * j + wave) + lane / LPR, c = (lane % LPR) ^ ((r & 3) << 2);
         offa[j] = (uint32_t)(r * a.ldd + c * 8) * 2u;
+        if constexpr (RAG) offa[j] |= m0 + c * 8 < a.M ? 0u : BUF_OOB;
     }
 #pragma unroll
     for (int j = 0; j < JJ; ++j) {
-        const int r = 2 * (NW * j + wave) + (lane >> 5), c = (lane & 31) ^ ((r & 3) << 2);
+        const int r = RPBB * (NW * j + wave) + lane / LPRB, c = (lane % LPRB) ^ ((r & 3) << 2);
         offb[j] = (uint32_t)(r * a.ldx + c * 8) * 2u;
+        if constexpr (RAG) offb[j] |= n0 + c * 8 < a.N ? 0u : BUF_OOB;
     }
     // packed x_hat: this thread's decode row and column run, and its flat element offset in a slab
     const int br = tid >> 3, bj = tid & 7;
@@ -423,6 +439,27 @@ __global__ __launch_bounds__(64 * NW, 1) void dw_gemm_v2_kernel(DwArgs a) {
         kt = min(kt, kt1 - 1);
         const char* ga = (const char*)(a.dy + kt * V2_BK * a.ldd + m0);
         char* da = sa + opaque0;
+        if constexpr (RAG) {
+            // rows of this slab that exist: a lane's offset in row r is at least r * ld * 2
+            const uint32_t rows = (uint32_t)min((int64_t)V2_BK, a.K - kt * V2_BK);
+            const char* gb = (const char*)(a.xh + kt * V2_BK * a.ldx + n0);
+            char* db = sb + opaque0;
+            const __amdgpu_buffer_rsrc_t ra =
+                __builtin_amdgcn_make_buffer_rsrc((void*)ga, (short)0, (int)(rows * (uint32_t)a.ldd * 2u), 0x00020000);
+            const __amdgpu_buffer_rsrc_t rb =
+                __builtin_amdgcn_make_buffer_rsrc((void*)gb, (short)0, (int)(rows * (uint32_t)a.ldx * 2u), 0x00020000);
+#pragma unroll
+            for (int j = 0; j < JA; ++j) {
+                const uint32_t off = offa[j];
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_void_t*)(da + (NW * j + wave) * 1024), 16, off, 0, 0, 0);
+            }
+#pragma unroll
+            for (int j = 0; j < JJ; ++j) {
+                const uint32_t off = offb[j];
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_void_t*)(db + (NW * j + wave) * 1024), 16, off, 0, 0, 0);
+            }
+            return;
+        }
 #pragma unroll
         for (int j = 0; j < JA; ++j)
             __builtin_amdgcn_global_load_lds((gbl_void_t*)(ga + offa[j]), (lds_void_t*)(da + (NW * j + wave) * 1024),
@@ -515,7 +552,7 @@ __global__ __launch_bounds__(64 * NW, 1) void dw_gemm_v2_kernel(DwArgs a) {
 #pragma unroll
         for (int ii = 0; ii < TMW; ++ii) fa[ii] = v2_frag<RA>(sa, kk, wm * RW + ii * 32, lane);
 #pragma unroll
-        for (int jj = 0; jj < TNW; ++jj) fb[jj] = v2_frag<V2_ROWB>(sb, kk, wn * CW + jj * 32, lane);
+        for (int jj = 0; jj < TNW; ++jj) fb[jj] = v2_frag<RB>(sb, kk, wn * CW + jj * 32, lane);
     };
     // bias-gradient pairs of fragment row ii
     auto db_row = [&](const uint4* fa, int ii) {
@@ -618,23 +655,46 @@ __global__ __launch_bounds__(64 * NW, 1) void dw_gemm_v2_kernel(DwArgs a) {
     __builtin_amdgcn_s_waitcnt(0);
 
     float* P = a.partial + (int64_t)split * a.M * a.N;
-#pragma unroll
-    for (int i = 0; i < TMW; ++i)
+    if constexpr (RAG) {
+        // rows past M lie past the end of the split's partial matrix, columns past N load the mask: neither
+        // is stored (and no branch per element)
+        const int64_t left = ((a.M - m0) * a.N - n0) * 4;
+        const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(
+            (void*)(P + m0 * a.N + n0), (short)0, (int)min(left, (int64_t)0x7FFFFF00), 0x00020000);
+        const uint32_t rowb = (uint32_t)a.N * 4u;
 #pragma unroll
         for (int j = 0; j < TNW; ++j) {
-            const int64_t col = n0 + wn * CW + j * 32 + (lane & 31);
+            const int64_t col = wn * CW + j * 32 + (lane & 31);
+            const uint32_t off = ((uint32_t)(wm * RW + 4 * (lane >> 5)) * rowb + (uint32_t)col * 4u) |
+                                 (n0 + col < a.N ? 0u : BUF_OOB);
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int64_t row = m0 + wm * RW + i * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-                P[row * a.N + col] = acc[i][j][v];
-            }
+            for (int i = 0; i < TMW; ++i)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    const uint32_t o = off + (uint32_t)(i * 32 + 8 * (v >> 2) + (v & 3)) * rowb;
+                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[i][j][v]), rp, o, 0, 0);
+                }
         }
+    } else {
+#pragma unroll
+        for (int i = 0; i < TMW; ++i)
+#pragma unroll
+            for (int j = 0; j < TNW; ++j) {
+                const int64_t col = n0 + wn * CW + j * 32 + (lane & 31);
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    const int64_t row = m0 + wm * RW + i * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+                    P[row * a.N + col] = acc[i][j][v];
+                }
+            }
+    }
     if (db_wave) {
         // lanes l and l + 32 hold the two token halves of column l % 32
 #pragma unroll
         for (int ii = 0; ii < TMW; ++ii) {
             const float other = __shfl_xor(dbacc[ii], 32);
-            if (lane < 32) a.db_partial[(int64_t)split * a.M + m0 + wm * RW + ii * 32 + lane] = dbacc[ii] + other;
+            const int64_t m = m0 + wm * RW + ii * 32 + lane;
+            if (lane < 32 && (!RAG || m < a.M)) a.db_partial[(int64_t)split * a.M + m] = dbacc[ii] + other;
         }
     }
 }
@@ -722,14 +782,31 @@ void launch_dw_reduce(const float* partial, int used, int64_t MN, float* out32, 
 
 // Output rows per workgroup of the pipelined kernel: 128 when 256 x 256 tiles would number 16 or
 // fewer (the split count, and with it the fp32 split partials written and read back, halves).
-int dw_tile_rows(int64_t M, int64_t N) { return (M / 256) * (N / 256) <= 16 ? 128 : 256; }
+int dw_tile_rows(int64_t M, int64_t N) { return ((M + 255) / 256) * ((N + 255) / 256) <= 16 ? 128 : 256; }
 
+// Output columns per workgroup: 256, or 128 where the last 256-wide tile would be at most half full (ragged
+// N only; 256 x 128 tiles are not built)
+int dw_tile_cols(int64_t M, int64_t N) {
+    const int64_t over = N % 256;
+    return over > 0 && over <= 128 && dw_tile_rows(M, N) == 128 ? 128 : 256;
+}
+
+// K splits of a shape: the same for every kernel of it, so all of them split K at the same token
+// boundaries. At most one round of 256 workgroups (one per CU: 128 KB of LDS each). Within that a split more
+// takes a 1/S share off the K loop, slabs * t per workgroup (t = 0.77 us per 32-token slab of a 256-row tile, 0.4
+// of a 128-row one), and adds an fp32 partial matrix written and read back (8 M N bytes at about
+// 5 TB/s): least at S = sqrt(slabs * t * 5e6 / (8 M N)). Long sequences hit the first limit (ViT-B/16 at
+// batch 128: 7, 9 and 14 splits as before); with few tokens the partials had cost more than the product:
+// 1024 x 1024 over 333 tokens 24.0 -> 13.7 us (with the direct result below), 768 x 768 over 985 23.9 -> 15.7,
+// 3072 x 3072 over 4001 185 -> 105.
 int dw_splits(int64_t M, int64_t N, int64_t K) {
-    // the same for every kernel of a shape, so all of them split K at the same token boundaries
-    const int64_t tiles = std::max<int64_t>((M / dw_tile_rows(M, N)) * (N / BN), 1);
+    const int bmt = dw_tile_rows(M, N), bnt = dw_tile_cols(M, N);
+    const int64_t tiles = std::max<int64_t>(((M + bmt - 1) / bmt) * ((N + bnt - 1) / bnt), 1);
     const int64_t kts = (K + BK - 1) / BK;
-    // one round of at most 256 workgroups (one per CU: 128 KB of LDS each)
+    const double slabs = (double)(K + V2_BK - 1) / V2_BK, t = bmt == 256 ? 0.77 : 0.4;
+    const double best = std::sqrt(slabs * t * 5e6 / (8.0 * (double)M * (double)N));
     int64_t s = std::max<int64_t>(256 / tiles, 1);
+    s = std::min(s, std::max<int64_t>((int64_t)(best + 0.5), 1));
     s = std::min(s, kts);
     return (int)std::max<int64_t>(s, 1);
 }
@@ -741,6 +818,9 @@ int64_t dw_workspace_floats(int64_t M, int64_t N, int64_t K) {
 
 int launch_dw_gemm(DwArgs a, int mode, bool with_db, float* out32, uint16_t* out16, float* db, hipStream_t st) {
     const int splits = dw_splits(a.M, a.N, a.K);
+    // one split and an fp32 result: the only partial matrix is the result, written in place
+    const bool direct = splits == 1 && a.K > 0 && out32 && !out16;
+    if (direct) a.partial = out32;
     // the packed codes go through the pipelined kernel for 1/2/4 bits with DMA-aligned arrays
     // (codes 16-byte, scale/min 4-byte aligned); 8-bit codes through the register-decoding kernel
     const bool v2_packed = mode == DW_B_PACKED && (a.bits == 1 || a.bits == 2 || a.bits == 4) &&
@@ -749,19 +829,25 @@ int launch_dw_gemm(DwArgs a, int mode, bool with_db, float* out32, uint16_t* out
     // (the pipelined kernel keeps a slab's lane offsets in 32 bits: 32 rows of either operand
     // must span less than 4 GiB)
     const bool v2_offsets = a.ldd < ((int64_t)1 << 26) && a.ldx < ((int64_t)1 << 26) && a.N < ((int64_t)1 << 26);
-    if ((mode == DW_B_BF16 || v2_packed) && v2_offsets && a.K > 0 && a.K % V2_BK == 0) {
+    const bool ragged = a.K % V2_BK != 0 || a.M % BM != 0 || a.N % BN != 0;
+    // (the ragged instances keep 32 rows of either operand and 256 rows of the partial matrix in a buffer
+    // resource's 31-bit range)
+    const bool v2_ragged = mode == DW_B_BF16 && a.ldd < ((int64_t)1 << 24) && a.ldx < ((int64_t)1 << 24) &&
+                           a.N < ((int64_t)1 << 20);
+    if ((mode == DW_B_BF16 || v2_packed) && (ragged ? v2_ragged : v2_offsets) && a.K > 0) {
         // the transpose-free kernel: 32-token tiles, split at the same token boundaries as the
         // 64-token kernel, so both accumulate the same 16-token MFMA steps in the same order
         // (K % 32 == 0 and N % 256 == 0 make the group count K N / g even, so the scale/min dword
         // loads stay inside their arrays)
-        const int64_t kts = a.K / V2_BK;
+        const int64_t kts = (a.K + V2_BK - 1) / V2_BK;
         const int64_t kts64 = (a.K + BK - 1) / BK;
         a.kt_per_split = std::max<int64_t>((kts64 + splits - 1) / splits, 1) * (BK / V2_BK);
         const int used = (int)((kts + a.kt_per_split - 1) / a.kt_per_split);
         a.splits = used;
-        a.db_partial = a.partial + (int64_t)splits * a.M * a.N;
+        a.db_partial = direct ? db : a.partial + (int64_t)splits * a.M * a.N;
         const int bmt = dw_tile_rows(a.M, a.N);
-        const int64_t W = (a.M / bmt) * (a.N / BN) * used;
+        const int bnt = dw_tile_cols(a.M, a.N);
+        const int64_t W = ((a.M + bmt - 1) / bmt) * ((a.N + bnt - 1) / bnt) * used;
         const dim3 grid((unsigned)(DW_XCDS * ((W + DW_XCDS - 1) / DW_XCDS)));
 #define DOPT_DW2T(BITS_, BMT_)                                                                                     \
     do {                                                                                                           \
@@ -773,20 +859,34 @@ int launch_dw_gemm(DwArgs a, int mode, bool with_db, float* out32, uint16_t* out
         if (bmt == 128) DOPT_DW2T(BITS_, 128);   \
         else DOPT_DW2T(BITS_, 256);              \
     } while (0)
-        if (mode == DW_B_BF16) DOPT_DW2(0);
+#define DOPT_DW2R(BMT_, BNT_)                                                                                          \
+    do {                                                                                                               \
+        if (with_db) hipLaunchKernelGGL((dw_gemm_v2_kernel<0, true, 4, BMT_, BNT_, true>), grid, dim3(256), 0, st, a);  \
+        else hipLaunchKernelGGL((dw_gemm_v2_kernel<0, false, 4, BMT_, BNT_, true>), grid, dim3(256), 0, st, a);         \
+    } while (0)
+        if (ragged && bmt == 256) DOPT_DW2R(256, 256);
+        else if (ragged && bnt == 256) DOPT_DW2R(128, 256);
+        else if (ragged) DOPT_DW2R(128, 128);
+        else if (mode == DW_B_BF16) DOPT_DW2(0);
         else if (a.bits == 1) DOPT_DW2(1);
         else if (a.bits == 2) DOPT_DW2(2);
         else DOPT_DW2(4);
+#undef DOPT_DW2R
 #undef DOPT_DW2
 #undef DOPT_DW2T
-        launch_dw_reduce(a.partial, used, a.M * a.N, out32, out16, a.db_partial, a.M, with_db ? db : nullptr, st);
+        if (!direct) launch_dw_reduce(a.partial, used, a.M * a.N, out32, out16, a.db_partial, a.M, with_db ? db : nullptr, st);
+        return 0;
+    }
+    if (a.M % BM != 0 || a.N % BN != 0) {
+        if (a.K > 0) return -1;  // outside the ragged instances' offsets
+        launch_dw_reduce(a.partial, 0, a.M * a.N, out32, out16, a.partial, a.M, with_db ? db : nullptr, st);
         return 0;
     }
     const int64_t kts = (a.K + BK - 1) / BK;
     a.kt_per_split = std::max<int64_t>((kts + splits - 1) / splits, 1);
     const int used = kts ? (int)((kts + a.kt_per_split - 1) / a.kt_per_split) : 0;  // splits with work
     a.splits = used;
-    a.db_partial = a.partial + (int64_t)splits * a.M * a.N;
+    a.db_partial = direct ? db : a.partial + (int64_t)splits * a.M * a.N;
     const int tiles = (int)((a.M / BM) * (a.N / BN));
     // ids: 8 XCDs x ceil(W / 8) slots; slots past W exit at once
     const int64_t W = (int64_t)tiles * used;
@@ -803,7 +903,7 @@ int launch_dw_gemm(DwArgs a, int mode, bool with_db, float* out32, uint16_t* out
 #undef DOPT_DW_DB
 #undef DOPT_DW
     }
-    launch_dw_reduce(a.partial, used, a.M * a.N, out32, out16, a.db_partial, a.M, with_db ? db : nullptr, st);
+    if (!direct) launch_dw_reduce(a.partial, used, a.M * a.N, out32, out16, a.db_partial, a.M, with_db ? db : nullptr, st);
     return 0;
 }
 

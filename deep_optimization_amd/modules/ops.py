@@ -14,7 +14,8 @@ x_hat + upsample(avgpool(x)), about x plus its low-pass (ops.py:245-264, :457-47
 module_utils.py:86-102); this is kept as the reference computes it, for parity.
 
 The Linear weight gradient ``dy^T . x_hat`` (and the bias gradient) runs on the gfx950 kernel
-behind ``act_lib::dw_gemm`` when dy is bf16 and both feature counts are multiples of 256; the
+behind ``act_lib::dw_gemm`` when dy is bf16 and both feature counts are multiples of 256 (and on
+``act_lib::dw_gemm_any`` for other multiples of 8 where it is the faster one); the
 per-layer meta key ``dw_fused_unpack`` (default False) makes that kernel decode the packed codes
 itself instead of reading the dequantized x_hat.
 
@@ -34,7 +35,7 @@ from torch.amp import custom_bwd, custom_fwd
 from torch.autograd import Function
 from torch.nn.modules.utils import _pair, _single, _triple
 
-from ..dw_lib import dw_gemm_supported
+from ..dw_lib import dw_any_preferred, dw_gemm_supported
 from .module_utils import unified_dequantize, unified_quantize
 
 
@@ -177,6 +178,11 @@ class _DOLinear(Function):
                 input = unified_dequantize((q0, q1, q2), ctx.q_inputs_meta, input_l)
                 dw, db = torch.ops.act_lib.dw_gemm(dy_flat, input.reshape(-1, C_in), None, None, None, C_in, 0, 0,
                                                    has_bias, out_dtype)
+        elif dy.dtype == torch.bfloat16 and dw_any_preferred(C_out, C_in, dy_flat.shape[0], has_bias):
+            # other feature counts: the same kernel's ragged instances
+            out_dtype = ctx.w_dtype if ctx.w_dtype in (torch.float32, torch.bfloat16) else torch.float32
+            input = unified_dequantize((q0, q1, q2), ctx.q_inputs_meta, input_l)
+            dw, db = torch.ops.act_lib.dw_gemm_any(dy_flat, input.reshape(-1, C_in), has_bias, out_dtype)
         else:
             input = unified_dequantize((q0, q1, q2), ctx.q_inputs_meta, input_l).to(dy.dtype)
             dw = dy_flat.t().mm(input.reshape(-1, C_in))
