@@ -9,15 +9,20 @@
 //
 // Errors: bad bits raise ValueError (TORCH_CHECK_VALUE), as act_triton_kernel.py:329-330 and
 // act_lib._bits_consts do; NotImplementedError where the Python implementations raise it;
-// everything else RuntimeError. A device guard makes the tensors' device current for the call.
+// everything else RuntimeError. A device guard makes the tensors' device current for the call (the operators
+// whose Python implementation refuses tensors of another device refuse them here too).
 //
 // Operators: quant_pack, quant_pack_tiles, dequant_unpack, dequant_unpack_tiles,
 // quant_pack_triton, dequant_unpack_triton (AC/act_triton_kernel.py:336-395),
 // relu_fwd_fused_pack, relu_bwd_fused_unpack (AC/modules/activations/kernel_registration.py:42-94),
-// bn_train_fwd, bn_train_bwd (the compressed BatchNorm layers' one-call forward and backward).
+// bn_train_fwd, bn_train_bwd (the compressed BatchNorm layers' one-call forward and backward),
+// silu_fwd_quan_pack, silu_bwd_fused_dequan_unpack, gelu_bwd_fused_dequan_unpack
+// (AC/modules/activations/kernel_registration.py:148-237, :295-319), dw_gemm_any (the compressed Linear layer's
+// weight gradient), fp8_gemm_nt, fp8_linear.
 #include <ATen/ATen.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPFunctions.h>
 #include <torch/library.h>
 
 #include <cmath>
@@ -60,6 +65,15 @@ int meta_code(ScalarType t) { return t == ScalarType::Float ? DOPT_F32 : DOPT_BF
 
 void require_cuda(const Tensor& t) {
     TORCH_CHECK(t.device().is_cuda(), "act_lib operators run on HIP (cuda) tensors only");
+}
+
+// the C ABI launches on the calling thread's current device: where the Python implementation refuses tensors of
+// another device (act_lib._stream) instead of switching to it, so does the native one
+void require_current(const Tensor& t) {
+    const auto cur = c10::hip::current_device();
+    TORCH_CHECK(t.device().index() == cur, "act_lib operators launch on the current device (", (int)cur,
+                "); the tensors are on cuda:", (int)t.device().index(), ": call under torch.cuda.device(",
+                (int)t.device().index(), ")");
 }
 
 // contiguous with a 16-byte aligned base (the kernels use 128-bit accesses)
@@ -303,6 +317,201 @@ Tensor relu_bwd_fused_unpack(const Tensor& packed_in, const Tensor& dy_in, int64
     return dx;
 }
 
+// ---------------------------------------------------------------------------- SiLU / GELU layers
+void require_group(int64_t group_size) {
+    TORCH_CHECK(group_size > 0 && group_size < ((int64_t)1 << 31), "unsupported group size ", group_size);
+}
+
+// (N, G) of x.view(N, -1, group_size)
+std::pair<int64_t, int64_t> flat_groups(const Tensor& x, int64_t group_size) {
+    const int64_t N = x.size(0);
+    TORCH_CHECK(N > 0 && x.numel() % (N * group_size) == 0, "x of shape ", x.sizes(),
+                " does not split into [N, G, ", group_size, "] groups");
+    return {N, x.numel() / N / group_size};
+}
+
+// whether the reference groups x into s x s spatial tiles (tensor_act_reshape_utils.tile_layout_applies)
+bool tile_layout_applies(const Tensor& x, int64_t group_size) {
+    if (x.dim() != 4) return false;
+    const int64_t s = (int64_t)std::sqrt((double)group_size);  // exact: group sizes are below 2^31
+    if (x.size(2) % s || x.size(3) % s) return false;
+    TORCH_CHECK(s * s == group_size, "spatial tile grouping needs a square group size: group_size=", group_size,
+                " is not s*s although H=", x.size(2), " and W=", x.size(3), " are divisible by s=", s);
+    return true;
+}
+
+bool silu_alam(bool avg_alam, int64_t alam_bits, const char* where) {
+    TORCH_CHECK_NOT_IMPLEMENTED(!avg_alam || alam_bits == 1, where, ": avg_alam=True with alam_bits=", alam_bits,
+                                ": the reference's SiLU forward kernel cannot reshape the codes for alam_bits >= 2 "
+                                "(alam_bits = 1 is supported)");
+    return avg_alam;
+}
+
+std::tuple<Tensor, Tensor, Tensor, Tensor, int64_t, int64_t, int64_t, int64_t, bool, bool> silu_fwd_quan_pack(
+    const Tensor& x_in, int64_t bits, int64_t group_size, bool avg_alam, int64_t alam_bits, bool /*pack_only*/) {
+    silu_alam(avg_alam, alam_bits, "silu_fwd_quan_pack");  // alam_bits = 1: the plain codes
+    require_group(group_size);
+    const bool tiles = tile_layout_applies(x_in, group_size);
+    int64_t N, G, nh = 0, nw = 0;
+    int64_t shape[4] = {0, 0, 0, 0};
+    if (tiles) {
+        std::tie(N, G) = tile_groups(x_in.sizes(), group_size);
+        const int64_t s = (int64_t)std::llround(std::sqrt((double)group_size));
+        for (int i = 0; i < 4; ++i) shape[i] = x_in.size(i);
+        nh = shape[2] / s;
+        nw = shape[3] / s;
+    } else {
+        std::tie(N, G) = flat_groups(x_in, group_size);
+    }
+    const int64_t nwords = words_per_group(bits, group_size);
+    TORCH_CHECK(x_in.scalar_type() == ScalarType::BFloat16 || x_in.scalar_type() == ScalarType::Float,
+                "fused activation quant-pack: input must be bfloat16 or float32, got ", x_in.scalar_type());
+    require_cuda(x_in);
+    require_current(x_in);
+    const Tensor x = aligned(x_in);
+    const auto bf16 = x.options().dtype(at::kBFloat16);
+    Tensor y = at::empty(x.sizes(), bf16);
+    Tensor packed = at::empty({N * G, nwords}, x.options().dtype(at::kInt));
+    Tensor scale = at::empty({N * G}, bf16), xmin = at::empty({N * G}, bf16);
+    check(dopt_act_quant_pack(x.data_ptr(), dtype_code(x.scalar_type(), "act_quant_pack"), DOPT_ACT_SILU, N * G,
+                              (int)group_size, (int)bits, tiles ? shape : nullptr, y.data_ptr(),
+                              (uint32_t*)packed.data_ptr(), scale.data_ptr(), xmin.data_ptr(), DOPT_BF16, stream_of(x)),
+          "act_quant_pack");
+    return {y, packed, scale, xmin, N, G, nh, nw, false, tiles};
+}
+
+Tensor act_dequant_mul(const Tensor& packed_in, const Tensor& dy_in, const Tensor& scale_in, const Tensor& xmin_in,
+                       int64_t bits, int64_t n_groups, int64_t group_size, const int64_t* tile, bool noise) {
+    const int64_t nwords = words_per_group(bits, group_size);
+    require_group(group_size);
+    TORCH_CHECK(dy_in.scalar_type() == ScalarType::BFloat16 || dy_in.scalar_type() == ScalarType::Float,
+                "fused activation backward: dy must be bfloat16 or float32, got ", dy_in.scalar_type());
+    TORCH_CHECK((scale_in.scalar_type() == ScalarType::Float || scale_in.scalar_type() == ScalarType::BFloat16) &&
+                    xmin_in.scalar_type() == scale_in.scalar_type(),
+                "fused activation backward: scale and min must both be float32 or both bfloat16");
+    TORCH_CHECK(dy_in.numel() == n_groups * group_size, "fused activation backward: dy has ", dy_in.numel(),
+                " elements, expected ", n_groups * group_size);
+    TORCH_CHECK(scale_in.numel() == n_groups && xmin_in.numel() == n_groups &&
+                    packed_in.numel() * packed_in.element_size() == n_groups * nwords * 4,
+                "fused activation backward: packed / scale / min do not hold ", n_groups, " groups");
+    require_cuda(packed_in);
+    require_cuda(dy_in);
+    require_cuda(scale_in);
+    require_cuda(xmin_in);
+    require_current(dy_in);
+    const Tensor packed = aligned(packed_in), dy = aligned(dy_in);
+    const Tensor scale = scale_in.contiguous(), xmin = xmin_in.contiguous();
+    Tensor dx = at::empty(dy.sizes(), dy.options().dtype(at::kBFloat16));
+    const int meta = meta_code(scale.scalar_type()), dyc = dtype_code(dy.scalar_type(), "act_dequant_mul");
+    const auto* codes = (const uint32_t*)packed.data_ptr();
+    check(noise ? dopt_act_dequant_mul_alam(codes, scale.data_ptr(), xmin.data_ptr(), meta, n_groups, (int)group_size,
+                                            (int)bits, tile, dy.data_ptr(), dyc, kAlamSeed, dx.data_ptr(), stream_of(dy))
+                : dopt_act_dequant_mul(codes, scale.data_ptr(), xmin.data_ptr(), meta, n_groups, (int)group_size,
+                                       (int)bits, tile, dy.data_ptr(), dyc, dx.data_ptr(), stream_of(dy)),
+          "act_dequant_mul");
+    return dx;
+}
+
+Tensor gelu_bwd_fused_dequan_unpack(const Tensor& packed, const Tensor& dy, const Tensor& scale, const Tensor& xmin,
+                                    int64_t bits, int64_t N, int64_t G, int64_t group_size) {
+    return act_dequant_mul(packed, dy, scale, xmin, bits, N * G, group_size, nullptr, false);
+}
+
+Tensor silu_bwd_fused_dequan_unpack(const Tensor& packed, const Tensor& dy, const Tensor& scale, const Tensor& xmin,
+                                    int64_t bits, int64_t N, int64_t G, int64_t group_size, bool /*pack_only*/,
+                                    int64_t /*new_H*/, int64_t /*new_W*/, bool /*padding_eligibility*/,
+                                    bool reshape_eligibility, bool avg_alam, int64_t alam_bits) {
+    const bool noise = silu_alam(avg_alam, alam_bits, "silu_bwd_fused_dequan_unpack");
+    int64_t shape[4] = {0, 0, 0, 0};
+    if (reshape_eligibility) {
+        TORCH_CHECK(dy.dim() == 4, "silu_bwd_fused_dequan_unpack: the tile layout expects a 4-D dy, got ", dy.sizes());
+        for (int i = 0; i < 4; ++i) shape[i] = dy.size(i);
+    }
+    return act_dequant_mul(packed, dy, scale, xmin, bits, N * G, group_size, reshape_eligibility ? shape : nullptr, noise);
+}
+
+// ---------------------------------------------------------------------------- Linear weight gradient
+std::tuple<Tensor, std::optional<Tensor>> dw_gemm_any(const Tensor& dy_in, const Tensor& x_in, bool bias_grad,
+                                                      ScalarType out_dtype) {
+    require_cuda(dy_in);
+    require_cuda(x_in);
+    TORCH_CHECK(dy_in.dim() == 2 && x_in.dim() == 2 && dy_in.size(0) == x_in.size(0) &&
+                    dy_in.scalar_type() == ScalarType::BFloat16 && x_in.scalar_type() == ScalarType::BFloat16,
+                "dw_gemm_any: dy and x_hat must be bf16 [K, M] and [K, N] matrices, got ", dy_in.sizes(), " ",
+                dy_in.scalar_type(), " and ", x_in.sizes(), " ", x_in.scalar_type());
+    TORCH_CHECK(out_dtype == ScalarType::Float || out_dtype == ScalarType::BFloat16,
+                "dw_gemm_any: out_dtype must be float32 or bfloat16, got ", out_dtype);
+    require_current(dy_in);
+    const int64_t K = dy_in.size(0), M = dy_in.size(1), N = x_in.size(1);
+    const Tensor dy = aligned(dy_in), x = aligned(x_in);
+    const auto f32 = dy.options().dtype(at::kFloat);
+    const int64_t floats = dopt_dw_gemm_any_workspace_floats(M, N, K);
+    Tensor ws = at::empty({floats > 4 ? floats : 4}, f32);
+    Tensor dw = at::empty({M, N}, dy.options().dtype(out_dtype));
+    std::optional<Tensor> db;
+    if (bias_grad) db = at::empty({M}, f32);
+    const bool wide = out_dtype == ScalarType::Float;
+    check(dopt_dw_gemm_any(dy.data_ptr(), M, x.data_ptr(), N, M, N, K, ws.data_ptr<float>(),
+                           wide ? dw.data_ptr<float>() : nullptr, wide ? nullptr : dw.data_ptr(),
+                           db ? db->data_ptr<float>() : nullptr, stream_of(dy)),
+          "dw_gemm_any");
+    return {dw, db};
+}
+
+// ---------------------------------------------------------------------------- FP8 GEMM
+Tensor fp8_gemm_nt(const Tensor& a_in, const Tensor& b_in, double out_scale) {
+    TORCH_CHECK(a_in.scalar_type() == ScalarType::Float8_e4m3fn && b_in.scalar_type() == ScalarType::Float8_e4m3fn,
+                "fp8_gemm_nt expects torch.float8_e4m3fn operands");
+    TORCH_CHECK(a_in.dim() == 2 && b_in.dim() == 2 && a_in.size(1) == b_in.size(1), "fp8_gemm_nt: shapes ",
+                a_in.sizes(), " x ", b_in.sizes(), "^T do not contract");
+    require_cuda(a_in);
+    require_cuda(b_in);
+    require_current(a_in);
+    const Tensor a = aligned(a_in), b = aligned(b_in);
+    const int64_t M = a.size(0), K = a.size(1), N = b.size(0);
+    Tensor c = at::empty({M, N}, a.options().dtype(at::kBFloat16));
+    check(dopt_fp8_gemm_nt((const uint8_t*)a.data_ptr(), (const uint8_t*)b.data_ptr(), M, N, K, K, K, (float)out_scale,
+                           c.data_ptr(), N, stream_of(a)),
+          "fp8_gemm_nt");
+    return c;
+}
+
+// an operand as the GEMM reads it (act_lib._kmajor): rows K-contiguous, 16-byte aligned, row stride a multiple
+// of 16; in place when it already is, else packed into a fresh [rows, k_pad] buffer with zero padding columns
+std::pair<Tensor, int64_t> kmajor(const Tensor& t, int64_t rows, int64_t k, int64_t stride_r, int64_t stride_k,
+                                  int64_t k_pad) {
+    if (stride_k == 1 && k == k_pad && stride_r % 16 == 0 && k <= stride_r && stride_r < (1 << 23) &&
+        reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0)
+        return {t, stride_r};
+    const auto bytes = t.options().dtype(at::kByte);
+    Tensor out = k_pad != k ? at::zeros({rows, k_pad}, bytes) : at::empty({rows, k_pad}, bytes);
+    check(dopt_fp8_pack_kmajor((const uint8_t*)t.data_ptr(), rows, k, stride_r, stride_k, (uint8_t*)out.data_ptr(), k_pad,
+                               stream_of(t)),
+          "fp8_pack_kmajor");
+    return {out, k_pad};
+}
+
+Tensor fp8_linear(const Tensor& a, const Tensor& b, double out_scale) {
+    TORCH_CHECK(a.scalar_type() == ScalarType::Float8_e4m3fn && b.scalar_type() == ScalarType::Float8_e4m3fn,
+                "fp8_linear expects torch.float8_e4m3fn operands");
+    TORCH_CHECK(a.dim() == 2 && b.dim() == 2 && a.size(1) == b.size(0), "fp8_linear: shapes ", a.sizes(), " x ",
+                b.sizes(), " do not contract");
+    require_cuda(a);
+    require_cuda(b);
+    require_current(a);
+    const int64_t M = a.size(0), K = a.size(1), N = b.size(1);
+    Tensor c = at::empty({M, N}, a.options().dtype(at::kBFloat16));
+    if (M == 0 || N == 0) return c;
+    if (K == 0) return c.zero_();
+    const int64_t k_pad = (K + 15) / 16 * 16;
+    const auto [ta, lda] = kmajor(a, M, K, a.stride(0), a.stride(1), k_pad);
+    const auto [tb, ldb] = kmajor(b, N, K, b.stride(1), b.stride(0), k_pad);
+    check(dopt_fp8_gemm_nt((const uint8_t*)ta.data_ptr(), (const uint8_t*)tb.data_ptr(), M, N, k_pad, lda, ldb,
+                           (float)out_scale, c.data_ptr(), N, stream_of(a)),
+          "fp8_linear");
+    return c;
+}
+
 // ---------------------------------------------------------------------------- BatchNorm layers
 int64_t bn_group(int64_t block) {
     const int64_t g = block / 2;
@@ -444,4 +653,10 @@ TORCH_LIBRARY_IMPL(act_lib, CUDA, m) {
     m.impl("relu_bwd_fused_unpack", &relu_bwd_fused_unpack);
     m.impl("bn_train_fwd", &bn_train_fwd);
     m.impl("bn_train_bwd", &bn_train_bwd);
+    m.impl("silu_fwd_quan_pack", &silu_fwd_quan_pack);
+    m.impl("silu_bwd_fused_dequan_unpack", &silu_bwd_fused_dequan_unpack);
+    m.impl("gelu_bwd_fused_dequan_unpack", &gelu_bwd_fused_dequan_unpack);
+    m.impl("dw_gemm_any", &dw_gemm_any);
+    m.impl("fp8_gemm_nt", &fp8_gemm_nt);
+    m.impl("fp8_linear", &fp8_linear);
 }

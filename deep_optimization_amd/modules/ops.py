@@ -14,15 +14,15 @@ x_hat + upsample(avgpool(x)), about x plus its low-pass (ops.py:245-264, :457-47
 module_utils.py:86-102); this is kept as the reference computes it, for parity.
 
 The Linear weight gradient ``dy^T . x_hat`` (and the bias gradient) runs on the gfx950 kernel
-behind ``act_lib::dw_gemm`` when dy is bf16 and both feature counts are multiples of 256 (and on
-``act_lib::dw_gemm_any`` for other multiples of 8 where it is the faster one); the
+behind ``act_lib::dw_gemm_any`` when dy is bf16 and both feature counts are multiples of 256, or
+multiples of 8 where it is the faster one; for multiples of 256 the
 per-layer meta key ``dw_fused_unpack`` (default False) makes that kernel decode the packed codes
-itself instead of reading the dequantized x_hat.
+itself (``act_lib::dw_gemm``) instead of reading the dequantized x_hat.
 
 Differences from the reference:
   * ``_DOLinear`` takes the bias and applies it (the reference calls ``F.linear(input, W, None)``
     and never trains the bias, ops.py:481); its gradient is ``dy`` summed over the rows;
-  * on the dw_gemm path the weight gradient comes back in the weight's dtype (fp32 master
+  * on that path the weight gradient comes back in the weight's dtype (fp32 master
     weights get an fp32 gradient; the reference's is bf16 under autocast);
   * the Conv Functions take an optional bias the same way (the reference's DOConv layers are
     built with ``bias=False``).
@@ -165,24 +165,22 @@ class _DOLinear(Function):
             dy = dy.to(dt)
         C_in, C_out = input_shape[-1], dy.shape[-1]
         dy_flat = dy.reshape(-1, C_out)
-        if dy.dtype == torch.bfloat16 and dw_gemm_supported(C_out, C_in):
+        out_dtype = ctx.w_dtype if ctx.w_dtype in (torch.float32, torch.bfloat16) else torch.float32
+        kernel = dy.dtype == torch.bfloat16
+        from_codes = ctx.fused_unpack and q1.dtype == torch.bfloat16 and dw_gemm_supported(C_out, C_in)
+        if kernel and from_codes:
             # weight (and bias) gradient on the gfx950 split-K GEMM for K-outer operands, in the
-            # weight's precision; x_hat is either dequantized first or decoded inside the GEMM
-            out_dtype = ctx.w_dtype if ctx.w_dtype in (torch.float32, torch.bfloat16) else torch.float32
-            if ctx.fused_unpack and q1.dtype == torch.bfloat16:
-                bits, group_size = ctx.q_inputs_meta[0], ctx.q_inputs_meta[2]
-                dw, db = torch.ops.act_lib.dw_gemm(dy_flat, None, q0, q1, q2, C_in, bits, group_size, has_bias,
-                                                   out_dtype)
-                input = None
-            else:
-                input = unified_dequantize((q0, q1, q2), ctx.q_inputs_meta, input_l)
-                dw, db = torch.ops.act_lib.dw_gemm(dy_flat, input.reshape(-1, C_in), None, None, None, C_in, 0, 0,
-                                                   has_bias, out_dtype)
-        elif dy.dtype == torch.bfloat16 and dw_any_preferred(C_out, C_in, dy_flat.shape[0], has_bias):
-            # other feature counts: the same kernel's ragged instances
-            out_dtype = ctx.w_dtype if ctx.w_dtype in (torch.float32, torch.bfloat16) else torch.float32
+            # weight's precision, x_hat decoded inside the GEMM
+            bits, group_size = ctx.q_inputs_meta[0], ctx.q_inputs_meta[2]
+            dw, db = torch.ops.act_lib.dw_gemm(dy_flat, None, q0, q1, q2, C_in, bits, group_size, has_bias, out_dtype)
+        elif kernel and dw_any_preferred(C_out, C_in, dy_flat.shape[0], has_bias):
+            # the same GEMM over the dequantized x_hat (one native operator call, with or without full tiles)
             input = unified_dequantize((q0, q1, q2), ctx.q_inputs_meta, input_l)
             dw, db = torch.ops.act_lib.dw_gemm_any(dy_flat, input.reshape(-1, C_in), has_bias, out_dtype)
+        elif kernel and dw_gemm_supported(C_out, C_in):  # 2^20 features and more
+            input = unified_dequantize((q0, q1, q2), ctx.q_inputs_meta, input_l)
+            dw, db = torch.ops.act_lib.dw_gemm(dy_flat, input.reshape(-1, C_in), None, None, None, C_in, 0, 0, has_bias,
+                                               out_dtype)
         else:
             input = unified_dequantize((q0, q1, q2), ctx.q_inputs_meta, input_l).to(dy.dtype)
             dw = dy_flat.t().mm(input.reshape(-1, C_in))

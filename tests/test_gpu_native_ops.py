@@ -125,3 +125,92 @@ def test_error_classes():
                          torch.empty(0, device=DEV), 0.1, 128, 2, _lib.BN_QUANT)
     with pytest.raises(RuntimeError, match="relu"):
         ops.relu_fwd_fused_pack(torch.zeros(2, 64, device=DEV), False, False, 1, 64)
+
+
+def planes(kind, x, w):
+    """the layouts fp8_linear takes in place and packs: [rows, K] row major, a column-major view, a misaligned slice"""
+    K = x.shape[1]
+    if kind == "row":
+        return x.contiguous(), w.contiguous().t()
+    if kind == "col":
+        return x.t().contiguous().t(), w.t().contiguous()
+    return x[:, 3:K - 2], w[:, 3:K - 2].t()
+
+
+@pytest.mark.parametrize("kind", ["row", "col", "slice"])
+@pytest.mark.parametrize("M,N,K", [(1, 8, 16), (5, 130, 250), (129, 64, 512), (0, 64, 64), (64, 0, 64)])
+def test_fp8_ops(M, N, K, kind):
+    a, b = planes(kind, rnd((M, K), 1).to(torch.float8_e4m3fn), rnd((N, K), 2).to(torch.float8_e4m3fn))
+    same(ops.fp8_linear(a, b, 0.125), act_lib._fp8_linear(a, b, 0.125))
+    if K % 16 == 0 and kind == "row":
+        same(ops.fp8_gemm_nt(a, b.t(), 0.125), act_lib._fp8_gemm_nt(a, b.t(), 0.125))
+
+
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K", [(8, 16, 5), (264, 520, 333), (256, 512, 700), (768, 256, 0)])
+def test_dw_gemm_any(M, N, K, out_dtype):
+    """... and, with both feature counts multiples of 256, dw_gemm on the same x_hat."""
+    from deep_optimization_amd import dw_lib
+
+    dy, x = rnd((K, M), 1), rnd((K, N), 2)
+    for bias in (True, False):
+        got = ops.dw_gemm_any(dy, x, bias, out_dtype)
+        same(got, dw_lib._dw_gemm_any(dy, x, bias, out_dtype))
+        if M % 256 == 0 and N % 256 == 0:
+            same(got, dw_lib._dw_gemm(dy, x, None, None, None, N, 0, 0, bias, out_dtype))
+    same(ops.dw_gemm_any(dy.t().contiguous().t(), x, True, out_dtype), ops.dw_gemm_any(dy, x, True, out_dtype))
+
+
+@pytest.mark.parametrize("shape,g", [((2, 8, 32, 48), 256), ((2, 16, 14, 14), 64), ((4, 12, 256), 128)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_silu_and_gelu_ops(shape, g, dtype):
+    for bits in (1, 2, 4, 8):
+        x, dy = rnd(shape, bits, dtype), rnd(shape, bits + 9, dtype)
+        for alam in ((False, 0), (True, 1)):
+            got = ops.silu_fwd_quan_pack(x, bits, g, *alam, False)
+            same(got, act_lib._silu_fwd_quan_pack(x, bits, g, *alam, False))
+            y, packed, scale, xmin, N, G, nh, nw, pe, re = got
+            bwd = (packed, dy, scale, xmin, bits, N, G, g, False, nh, nw, pe, re, *alam)
+            same(ops.silu_bwd_fused_dequan_unpack(*bwd), act_lib._silu_bwd_fused_dequan_unpack(*bwd))
+            same(ops.silu_bwd_fused_dequan_unpack(packed, dy.transpose(-1, -2).contiguous().transpose(-1, -2), *bwd[2:]),
+                 act_lib._silu_bwd_fused_dequan_unpack(*bwd))
+        y, packed, scale, xmin, N, G = ops.gelu_fwd_fused_quan_pack(x, bits, g)
+        bwd = (packed, dy, scale, xmin, bits, N, G, g)
+        same(ops.gelu_bwd_fused_dequan_unpack(*bwd), act_lib._gelu_bwd_fused_dequan_unpack(*bwd))
+
+
+@pytest.mark.parametrize("name,args,error", [
+    ("silu_fwd_quan_pack", ((4, 8, 256), 3, 256, False, 0, False), ValueError),
+    ("silu_fwd_quan_pack", ((4, 8, 256), 2, 256, True, 2, False), NotImplementedError),
+    ("silu_fwd_quan_pack", ((4, 8, 256), 2, 192, False, 0, False), RuntimeError),
+    ("silu_fwd_quan_pack", ((4, 8, 32, 32), 2, 130, False, 0, False), RuntimeError),
+    ("silu_fwd_quan_pack", ((4, 8, 33, 33), 2, 130, False, 0, False), RuntimeError),
+])
+def test_silu_errors(name, args, error):
+    """the classes that the Python implementations raise, on calls that the checks before any launch refuse"""
+    x = rnd(args[0], 1)
+    for f in (getattr(ops, name), getattr(act_lib, "_" + name)):
+        with pytest.raises(error):
+            f(x, *args[1:])
+
+
+def test_refused_operands():
+    a8, b8 = (rnd((64, 32), i).to(torch.float8_e4m3fn) for i in (1, 2))
+    x = rnd((64, 32), 3)
+    packed, s = torch.zeros((8, 16), dtype=torch.int32, device=DEV), torch.ones(8, device=DEV)
+    from deep_optimization_amd import dw_lib
+
+    bad = [(ops.fp8_linear, act_lib._fp8_linear, (a8, b8, 1.0)), (ops.fp8_linear, act_lib._fp8_linear, (x, a8.t(), 1.0)),
+           (ops.fp8_gemm_nt, act_lib._fp8_gemm_nt, (a8, b8.t(), 1.0)),
+           (ops.fp8_gemm_nt, act_lib._fp8_gemm_nt, (a8[:, :24], b8[:, :24], 1.0)),
+           (ops.dw_gemm_any, dw_lib._dw_gemm_any, (x.float(), x, True, torch.float32)),
+           (ops.dw_gemm_any, dw_lib._dw_gemm_any, (x, x[:32], True, torch.float32)),
+           (ops.dw_gemm_any, dw_lib._dw_gemm_any, (x, x, True, torch.float16)),
+           (ops.dw_gemm_any, dw_lib._dw_gemm_any, (x, x[:, :12], True, torch.float32)),
+           (ops.gelu_bwd_fused_dequan_unpack, act_lib._gelu_bwd_fused_dequan_unpack, (packed, x, s, s, 2, 4, 4, 256)),
+           (ops.gelu_bwd_fused_dequan_unpack, act_lib._gelu_bwd_fused_dequan_unpack,
+            (packed, x, s, s.bfloat16(), 2, 4, 2, 256))]
+    for native, python, args in bad:
+        for f in (native, python):
+            with pytest.raises(RuntimeError):
+                f(*args)
