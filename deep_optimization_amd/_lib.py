@@ -28,6 +28,8 @@ EXPORTS = (
     "dopt_pack_codes",
     "dopt_unpack_codes",
     "dopt_fp8_gemm_nt",
+    "dopt_fp8_gemm_kn",
+    "dopt_fp8_gemm_kn_preferred",
     "dopt_fp8_pack_kmajor",
     "dopt_relu_pack",
     "dopt_relu_unpack",
@@ -92,6 +94,10 @@ def lib() -> ctypes.CDLL:
         L.dopt_unpack_codes.restype = i32
         L.dopt_fp8_gemm_nt.argtypes = [vp, vp, i64, i64, i64, i64, i64, f32, vp, i64, vp]
         L.dopt_fp8_gemm_nt.restype = i32
+        L.dopt_fp8_gemm_kn.argtypes = [vp, vp, i64, i64, i64, i64, i64, i64, f32, vp, i64, vp]
+        L.dopt_fp8_gemm_kn.restype = i32
+        L.dopt_fp8_gemm_kn_preferred.argtypes = [i64, i64, i64]
+        L.dopt_fp8_gemm_kn_preferred.restype = i32
         L.dopt_fp8_pack_kmajor.argtypes = [vp, i64, i64, i64, i64, vp, i64, vp]
         L.dopt_fp8_pack_kmajor.restype = i32
         L.dopt_relu_pack.argtypes = [vp, i32, i64, i32, i32, vp, vp, vp]

@@ -448,7 +448,8 @@ def _fp8_linear(a, b, out_scale):
     a [M, K] @ b [K, N] with any strides -> bf16 [M, N] = out_scale * a @ b, fp32 accumulate. The
     GEMM reads both operands K-contiguous: an operand in another layout (b in its row-major [K, N]
     layout, a transposed view, unaligned rows, K not a multiple of 16) is first packed by
-    dopt_fp8_pack_kmajor (zero-padding K to a multiple of 16), the rest is read in place."""
+    dopt_fp8_pack_kmajor (zero-padding K to a multiple of 16), the rest is read in place. A row-major b
+    with 16-byte rows is read as it lies where that is the faster way (dopt_fp8_gemm_kn)."""
     if a.dtype != torch.float8_e4m3fn or b.dtype != torch.float8_e4m3fn:
         raise RuntimeError("fp8_linear expects torch.float8_e4m3fn operands")
     if a.dim() != 2 or b.dim() != 2 or a.shape[1] != b.shape[0]:
@@ -463,6 +464,13 @@ def _fp8_linear(a, b, out_scale):
         return c.zero_()
     k_pad = (K + 15) // 16 * 16
     ta, lda = _kmajor(a.view(torch.uint8), M, K, a.stride(0), a.stride(1), k_pad)
+    ldb = b.stride(0)
+    if b.stride(1) == 1 and ldb % 16 == 0 and N <= ldb < (1 << 23) and N % 16 == 0 and b.data_ptr() % 16 == 0 and \
+            _lib.lib().dopt_fp8_gemm_kn_preferred(M, N, k_pad):
+        rc = _lib.lib().dopt_fp8_gemm_kn(ta.data_ptr(), b.data_ptr(), M, N, k_pad, K, lda, ldb, float(out_scale),
+                                         c.data_ptr(), N, _stream(a))
+        _lib.check(rc, "fp8_linear")
+        return c
     tb, ldb = _kmajor(b.view(torch.uint8), N, K, b.stride(1), b.stride(0), k_pad)
     rc = _lib.lib().dopt_fp8_gemm_nt(ta.data_ptr(), tb.data_ptr(), M, N, k_pad, lda, ldb, float(out_scale),
                                      c.data_ptr(), N, _stream(a))

@@ -17,6 +17,9 @@ int launch_pack_codes(const int8_t* codes, uint32_t* out, uint64_t n_words, int 
 int launch_unpack_codes(const uint32_t* packed, int8_t* codes, uint64_t n_words, int bits, hipStream_t s);
 int launch_fp8_gemm_nt(const uint8_t* A, const uint8_t* B, int64_t M, int64_t N, int64_t K, int64_t lda,
                        int64_t ldb, float out_scale, uint16_t* C, int64_t ldc, hipStream_t s);
+int launch_fp8_gemm_kn(const uint8_t* A, const uint8_t* B, int64_t M, int64_t N, int64_t K, int64_t b_rows, int64_t lda,
+                       int64_t ldb, float out_scale, uint16_t* C, int64_t ldc, hipStream_t s);
+bool fp8_gemm_kn_preferred(int64_t M, int64_t N, int64_t K);
 int launch_fp8_pack(const uint8_t* src, int64_t rows, int64_t cols, int64_t stride_r, int64_t stride_c, uint8_t* dst,
                     int64_t ld_dst, hipStream_t s);
 int launch_relu_pack(const void* x, int dt, void* y, uint32_t* packed, uint64_t n, int bits, bool relu6, hipStream_t s);
@@ -399,6 +402,36 @@ int dopt_fp8_gemm_nt(const uint8_t* A, const uint8_t* B, int64_t M, int64_t N, i
     const int rc = dopt::launch_fp8_gemm_nt(A, B, M, N, K, lda, ldb, out_scale, (uint16_t*)C, ldc, (hipStream_t)stream);
     if (rc) return fail(DOPT_EUNSUPPORTED, "fp8 GEMM launch configuration unsupported");
     return hip_status("fp8_gemm launch");
+}
+
+int dopt_fp8_gemm_kn_preferred(int64_t M, int64_t N, int64_t K) {
+    return M > 0 && N > 0 && K > 0 && dopt::fp8_gemm_kn_preferred(M, N, K);
+}
+
+int dopt_fp8_gemm_kn(const uint8_t* A, const uint8_t* B, int64_t M, int64_t N, int64_t K, int64_t b_rows, int64_t lda,
+                     int64_t ldb, float out_scale, void* C, int64_t ldc, void* stream) {
+    if (M < 0 || N < 0 || K < 0) return fail(DOPT_EINVAL, "negative GEMM extent");
+    if (M == 0 || N == 0) return ok();
+    if (K == 0 || !A || !B || !C) return fail(DOPT_EINVAL, "fp8_gemm_kn: K is 0 or a pointer is null");
+    if (K % 16 || N % 16)
+        return fail(DOPT_EUNSUPPORTED, "fp8_gemm_kn needs K %% 16 == 0 and N %% 16 == 0, got K=%lld N=%lld", (long long)K,
+                    (long long)N);
+    if (b_rows > K || b_rows <= K - 16)
+        return fail(DOPT_EINVAL, "fp8_gemm_kn: B has K rows or up to 15 fewer, got %lld of %lld", (long long)b_rows,
+                    (long long)K);
+    if (lda < K || ldb < N || ldc < N || lda % 16 || ldb % 16 || !aligned16(A) || !aligned16(B) || ((uintptr_t)C & 1))
+        return fail(DOPT_EINVAL,
+                    "fp8_gemm_kn needs 16-byte aligned A and B, lda >= K and ldb >= N multiples of 16, a 2-byte aligned C "
+                    "and ldc >= N (got lda=%lld ldb=%lld ldc=%lld K=%lld N=%lld)",
+                    (long long)lda, (long long)ldb, (long long)ldc, (long long)K, (long long)N);
+    if (lda >= (1 << 23) || ldb >= (1 << 23))
+        return fail(DOPT_EINVAL, "fp8 GEMM row strides must be below 2^23 bytes (32-bit tile offsets), got %lld, %lld",
+                    (long long)lda, (long long)ldb);
+    if ((M + 31) / 32 * ((N + 63) / 64) >= ((int64_t)1 << 31))
+        return fail(DOPT_EINVAL, "fp8 GEMM output too large: %lld x %lld", (long long)M, (long long)N);
+    (void)hipGetLastError();
+    dopt::launch_fp8_gemm_kn(A, B, M, N, K, b_rows, lda, ldb, out_scale, (uint16_t*)C, ldc, (hipStream_t)stream);
+    return hip_status("fp8_gemm_kn launch");
 }
 
 int dopt_fp8_pack_kmajor(const uint8_t* src, int64_t rows, int64_t cols, int64_t stride_r, int64_t stride_c, uint8_t* dst,

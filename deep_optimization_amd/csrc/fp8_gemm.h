@@ -75,6 +75,7 @@ struct Fp8GemmArgs {
     float out_scale;
     uint32_t tiles_m, tiles_n;
     uint32_t vec_store;  // C 16-byte aligned with ldc % 8 == 0: whole chunks go out as 16-byte stores
+    int64_t b_rows;      // B given as [K, N] rows (fp8_gemm_mid.h): the rows it has, K or up to 15 fewer
 };
 
 template <int BM_, int BN_, int GROUP_M_, int SCHED_ = 1>

@@ -59,23 +59,26 @@ constexpr TileCost TILE_COST[T_COUNT] = {
     {256, 256, 5.0f, 0.95f, 1.45f, 2.5f},
 };
 
-int plan(int64_t M, int64_t N, int64_t K, int n_cu) {
+// the tile with the least estimate (kn: of those that read B as it lies in [K, N] rows) and that estimate
+int plan(int64_t M, int64_t N, int64_t K, int n_cu, bool kn, float* us_out) {
     const float nk = (float)((K + 127) / 128);
-    int best = T_256;
+    int best = kn ? T_128x128 : T_256;
     float least = 0.0f;
-    for (int t = T_COUNT - 1; t >= 0; --t) {
+    for (int t = kn ? T_128x128 : T_COUNT - 1; t >= (kn ? T_32x64 : 0); --t) {
         const TileCost& c = TILE_COST[t];
         if (t == T_SMALL && M > 16) continue;
         const int64_t tiles = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
         if (tiles >= ((int64_t)1 << 31)) continue;
         const float rounds = (float)((tiles + n_cu - 1) / n_cu);
-        const float step = c.rate * rounds > c.step ? c.rate * rounds : c.step;
+        const float rate = (kn ? 1.2f : 1.0f) * c.rate * rounds;  // the transposing reads: four per fragment for two
+        const float step = rate > c.step ? rate : c.step;
         const float us = c.start + nk * step + c.epilogue * rounds;
-        if (t == T_256 || us < least) {
+        if (t == best || us < least) {
             least = us;
             best = t;
         }
     }
+    *us_out = least;
     return best;
 }
 
@@ -85,8 +88,9 @@ int launch_fp8_gemm_nt(const uint8_t* A, const uint8_t* B, int64_t M, int64_t N,
                        int64_t ldb, float out_scale, uint16_t* C, int64_t ldc, hipStream_t s) {
     const int n_cu = device_cu_count();
     const Fp8GemmArgs p{A, B, C, M, N, K, lda, ldb, ldc, out_scale, 0, 0,
-                        (uint32_t)(ldc % 8 == 0 && ((uintptr_t)C & 15) == 0)};
-    switch (plan(M, N, K, n_cu)) {
+                        (uint32_t)(ldc % 8 == 0 && ((uintptr_t)C & 15) == 0), K};
+    float us;
+    switch (plan(M, N, K, n_cu, false, &us)) {
         case T_SMALL: return fp8_gemm_small_launch<1, 1, 8>(p, s);
         case T_32x64: return fp8_gemm_mid_launch<32, 64>(p, s);
         case T_64x64: return fp8_gemm_mid_launch<64, 64>(p, s);
@@ -95,6 +99,33 @@ int launch_fp8_gemm_nt(const uint8_t* A, const uint8_t* B, int64_t M, int64_t N,
         case T_128x128_NT: return fp8_gemm_launch<Fp8Gemm128>(A, B, M, N, K, lda, ldb, out_scale, C, ldc, s);
     }
     return fp8_gemm_persistent_launch<Fp8GemmDefault>(A, B, M, N, K, lda, ldb, out_scale, C, ldc, n_cu, s);
+}
+
+// B in [K, N] rows
+int launch_fp8_gemm_kn(const uint8_t* A, const uint8_t* B, int64_t M, int64_t N, int64_t K, int64_t b_rows, int64_t lda,
+                       int64_t ldb, float out_scale, uint16_t* C, int64_t ldc, hipStream_t s) {
+    const Fp8GemmArgs p{A, B, C, M, N, K, lda, ldb, ldc, out_scale, 0, 0,
+                        (uint32_t)(ldc % 8 == 0 && ((uintptr_t)C & 15) == 0), b_rows};
+    float us;
+    switch (plan(M, N, K, device_cu_count(), true, &us)) {
+        case T_32x64: return fp8_gemm_mid_launch<32, 64, true>(p, s);
+        case T_64x64: return fp8_gemm_mid_launch<64, 64, true>(p, s);
+        case T_128x64: return fp8_gemm_mid_launch<128, 64, true>(p, s);
+    }
+    return fp8_gemm_mid_launch<128, 128, true>(p, s);
+}
+
+// Whether reading B as it lies is estimated to be faster than packing it (a launch of about 3 us and its
+// bytes) for launch_fp8_gemm_nt. Both ways timed on 16 shapes from 1 x 4096 x 4096 to 8192^3; us, packed ->
+// as it lies: 985 x 768 x 1536 8.5 -> 5.5, 64 x 4096 x 4096 17.1 -> 6.7, 1024^3 7.8 -> 4.8, 2048^3
+// 18.0 -> 11.4, 8192 x 1024 x 1024 17.6 -> 15.3; the other way at 3000^3 (50.7 against 55.8) and 4096^3
+// (57.4 against 72.2), where the 256 x 256 tiles win.
+bool fp8_gemm_kn_preferred(int64_t M, int64_t N, int64_t K) {
+    const int n_cu = device_cu_count();
+    float kn, nt;
+    plan(M, N, K, n_cu, true, &kn);
+    plan(M, N, K, n_cu, false, &nt);
+    return kn < nt + 3.0f + (float)N * (float)K * (1.0f / 3.2e6f);
 }
 
 }  // namespace dopt

@@ -13,13 +13,23 @@
 //
 // LDS rows are the slab's 128 bytes; 16-byte chunk c of row r lies at c ^ f(r), f as in
 // fp8_gemm16_persistent_kernel (the same 16-row fragments).
+//
+// KN: B lies as [K, N] rows (a weight used as x @ w), N and its row stride multiples of 16 bytes. Its slab is
+// then 128 rows of BN bytes, loaded as they lie, and the operand reads transpose: ds_read_b64_tr_b8 hands 16
+// lanes an 8 x 16 block of bytes by columns, four of them make a fragment's 32 K bytes per lane (the K order of
+// the other form, so the sums are the same bit for bit). 16-byte chunk c of row k lies at c ^ g(k), so the 16
+// rows that 32 lanes read at once (8 i .. + 7 and 32 + 8 i .. + 7) fall into different banks. The form spares
+// the transposed copy of B, a launch of its own: 985 x 1536 x 768 took 3.8 us for it beside 7.1 for the GEMM.
 #pragma once
 
 #include "fp8_gemm.h"
 
 namespace dopt {
 
-template <int BM, int BN>
+typedef int v2i_t __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) v2i_t lds_v2i_t;
+
+template <int BM, int BN, bool KN>
 __global__ __launch_bounds__(256, 1) void fp8_gemm_mid_kernel(Fp8GemmArgs p) {
     constexpr int BK = 128, WM = BM / 2, WN = BN / 2, FM = WM / 16, FN = WN / 16;
     constexpr int LA = BM / 32, LB = BN / 32, LD = LA + LB;  // 1 KB loads per wave and slab
@@ -56,14 +66,29 @@ __global__ __launch_bounds__(256, 1) void fp8_gemm_mid_kernel(Fp8GemmArgs p) {
     const __amdgpu_buffer_rsrc_t ra =
         __builtin_amdgcn_make_buffer_rsrc((void*)(p.A + m0 * lda), (short)0, (int)GEMM_RANGE, 0x00020000);
     const __amdgpu_buffer_rsrc_t rb =
-        __builtin_amdgcn_make_buffer_rsrc((void*)(p.B + n0 * ldb), (short)0, (int)GEMM_RANGE, 0x00020000);
+        __builtin_amdgcn_make_buffer_rsrc((void*)(p.B + (KN ? 0 : n0 * ldb)), (short)0, (int)GEMM_RANGE, 0x00020000);
     uint32_t offa[LA], offb[LB];
 #pragma unroll
     for (int j = 0; j < LA; ++j)
         offa[j] = m0 + 32 * j + lrow < M ? (uint32_t)((32 * j + lrow) * lda + lchunk * 16) : GEMM_OOB;
+    if constexpr (KN) {
+        // load j of wave w fills rows k = RPL (4 j + w) + lane / CPR of CPR chunks, position lane % CPR <- chunk
+        // (lane % CPR) ^ g(k): g = k2 | k5 << 1 at 4 chunks a row, k1 | k2 << 1 | k5 << 2 at 8
+        constexpr int CPR = BN / 16, RPL = 64 / CPR;
+        static_assert(CPR == 4 || CPR == 8, "swizzles of 64- and 128-byte rows");
 #pragma unroll
-    for (int j = 0; j < LB; ++j)
-        offb[j] = n0 + 32 * j + lrow < N ? (uint32_t)((32 * j + lrow) * ldb + lchunk * 16) : GEMM_OOB;
+        for (int j = 0; j < LB; ++j) {
+            const int k = RPL * (4 * j + wave) + lane / CPR;
+            const int g = CPR == 4 ? ((k >> 2) & 1) | (((k >> 5) & 1) << 1)
+                                   : ((k >> 1) & 1) | (((k >> 2) & 1) << 1) | (((k >> 5) & 1) << 2);
+            const int col = ((lane & (CPR - 1)) ^ g) * 16;
+            offb[j] = n0 + col < N ? (uint32_t)(k * ldb + col) : GEMM_OOB;
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < LB; ++j)
+            offb[j] = n0 + 32 * j + lrow < N ? (uint32_t)((32 * j + lrow) * ldb + lchunk * 16) : GEMM_OOB;
+    }
     // (the LDS offsets carry a zero the compiler cannot see through: a read it could prove disjoint from
     // the one load it records per LDS object would wait for every load in flight)
     int opaque0;
@@ -78,11 +103,25 @@ __global__ __launch_bounds__(256, 1) void fp8_gemm_mid_kernel(Fp8GemmArgs p) {
             __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_void_t*)(da + wave * 1024 + j * 4096), 16, off, (int)k0,
                                                      0, 0);
         }
+        if constexpr (KN) {
+            // the slab's rows end with B's last: the buffer range covers what is left of it, so rows past it
+            // read zeros (a slab's offsets stay below 2^30, so a range cut to GEMM_RANGE covers whole slabs)
+            const int64_t left = (p.b_rows - 1 - (int64_t)k0) * ldb + N - n0;
+            const int range = left <= 0 ? 0 : left < (int64_t)GEMM_RANGE ? (int)left : (int)GEMM_RANGE;
+            const __amdgpu_buffer_rsrc_t rk =
+                __builtin_amdgcn_make_buffer_rsrc((void*)(p.B + (int64_t)k0 * ldb + n0), (short)0, range, 0x00020000);
 #pragma unroll
-        for (int j = 0; j < LB; ++j) {
-            const uint32_t off = offb[j] | past;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_void_t*)(db + wave * 1024 + j * 4096), 16, off, (int)k0,
-                                                     0, 0);
+            for (int j = 0; j < LB; ++j) {
+                const uint32_t off = offb[j];
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (lds_void_t*)(db + wave * 1024 + j * 4096), 16, off, 0, 0, 0);
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < LB; ++j) {
+                const uint32_t off = offb[j] | past;
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_void_t*)(db + wave * 1024 + j * 4096), 16, off,
+                                                         (int)k0, 0, 0);
+            }
         }
     };
 
@@ -99,9 +138,22 @@ __global__ __launch_bounds__(256, 1) void fp8_gemm_mid_kernel(Fp8GemmArgs p) {
         const v4u_t x1 = *(const v4u_t*)(s + (o + p1));
         return __builtin_bit_cast(v8i_t, __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7));
     };
+    // KN: fragment j is columns WN wn + 16 j + lane % 16; lane l names row 8 i + (l % 16) / 2 (+ 32 (l / 16)),
+    // half l % 2 of its 16 bytes, for the transposing read i
+    const int crow = 32 * (lane >> 4) + ((lane & 15) >> 1), chalf = 8 * (lane & 1);
+    const int cg = BN == 64 ? ((lane >> 3) & 1) | (((lane >> 4) & 1) << 1)
+                            : ((lane >> 2) & 1) | (((lane >> 3) & 1) << 1) | (((lane >> 4) & 1) << 2);
+    auto read_cols = [&](const uint8_t* s, int j) __attribute__((always_inline)) -> v8i_t {
+        const uint8_t* q = s + (crow * BN + (((wn * FN + j) ^ cg) << 4) + chalf);
+        const v2i_t x0 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i_t*)q);
+        const v2i_t x1 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i_t*)(q + 8 * BN));
+        const v2i_t x2 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i_t*)(q + 16 * BN));
+        const v2i_t x3 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i_t*)(q + 24 * BN));
+        return v8i_t{x0[0], x0[1], x1[0], x1[1], x2[0], x2[1], x3[0], x3[1]};
+    };
     auto read_frags = [&](Frags& f, const uint8_t* sa, const uint8_t* sb) __attribute__((always_inline)) {
 #pragma unroll
-        for (int j = 0; j < FN; ++j) f.b[j] = read_frag(sb, WN * wn + 16 * j);
+        for (int j = 0; j < FN; ++j) f.b[j] = KN ? read_cols(sb, j) : read_frag(sb, WN * wn + 16 * j);
 #pragma unroll
         for (int i = 0; i < FM; ++i) f.a[i] = read_frag(sa, WM * wm + 16 * i);
     };
@@ -124,7 +176,7 @@ __global__ __launch_bounds__(256, 1) void fp8_gemm_mid_kernel(Fp8GemmArgs p) {
         for (int i = 0; i < FM; ++i)
 #pragma unroll
             for (int j = 0; j < FN; ++j) acc[i][j] = mfma_fp8_16x16x128(cur.b[j], cur.a[i], acc[i][j]);
-        constexpr int NM = FM * FN, NR = 2 * (FM + FN);
+        constexpr int NM = FM * FN, NR = 2 * FM + (KN ? 4 : 2) * FN;
         constexpr int PER = (NR + NM - 1) / NM;
 #pragma unroll
         for (int q = 0; q < NM; ++q) {
@@ -192,11 +244,11 @@ __global__ __launch_bounds__(256, 1) void fp8_gemm_mid_kernel(Fp8GemmArgs p) {
     }
 }
 
-template <int BM, int BN>
+template <int BM, int BN, bool KN = false>
 inline int fp8_gemm_mid_launch(Fp8GemmArgs p, hipStream_t s) {
     p.tiles_m = (uint32_t)((p.M + BM - 1) / BM);
     p.tiles_n = (uint32_t)((p.N + BN - 1) / BN);
-    hipLaunchKernelGGL((fp8_gemm_mid_kernel<BM, BN>), dim3(p.tiles_m * p.tiles_n), dim3(256), 0, s, p);
+    hipLaunchKernelGGL((fp8_gemm_mid_kernel<BM, BN, KN>), dim3(p.tiles_m * p.tiles_n), dim3(256), 0, s, p);
     return 0;
 }
 

@@ -505,6 +505,13 @@ Tensor fp8_linear(const Tensor& a, const Tensor& b, double out_scale) {
     if (K == 0) return c.zero_();
     const int64_t k_pad = (K + 15) / 16 * 16;
     const auto [ta, lda] = kmajor(a, M, K, a.stride(0), a.stride(1), k_pad);
+    if (b.stride(1) == 1 && N % 16 == 0 && b.stride(0) % 16 == 0 && N <= b.stride(0) && b.stride(0) < (1 << 23) &&
+        reinterpret_cast<uintptr_t>(b.data_ptr()) % 16 == 0 && dopt_fp8_gemm_kn_preferred(M, N, k_pad)) {
+        check(dopt_fp8_gemm_kn((const uint8_t*)ta.data_ptr(), (const uint8_t*)b.data_ptr(), M, N, k_pad, K, lda, b.stride(0),
+                               (float)out_scale, c.data_ptr(), N, stream_of(a)),
+              "fp8_linear");
+        return c;
+    }
     const auto [tb, ldb] = kmajor(b, N, K, b.stride(1), b.stride(0), k_pad);
     check(dopt_fp8_gemm_nt((const uint8_t*)ta.data_ptr(), (const uint8_t*)tb.data_ptr(), M, N, k_pad, lda, ldb,
                            (float)out_scale, c.data_ptr(), N, stream_of(a)),

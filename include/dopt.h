@@ -154,6 +154,18 @@ int dopt_fp8_gemm_nt(const uint8_t* A, const uint8_t* B, int64_t M, int64_t N, i
                      int64_t lda, int64_t ldb, float out_scale, void* C, int64_t ldc, void* stream);
 
 /*
+ * The same product with B in row-major [K, N] rows (Triton_Linear's own layout), read as it lies:
+ * C[m][n] = bf16(out_scale * sum_k A[m][k] * B[k][n]). N % 16 == 0 and K % 16 == 0; B may have
+ * b_rows = K - 15 .. K rows (rows from b_rows to K count as zeros: A is then a copy padded to K columns).
+ * lda >= K and ldb >= N multiples of 16 and < 2^23, A and B 16-byte aligned, C as above.
+ * dopt_fp8_gemm_kn_preferred: 1 where this is estimated to be faster than packing B for
+ * dopt_fp8_gemm_nt first (outputs below the sizes that the 256 x 256 tiles need).
+ */
+int dopt_fp8_gemm_kn(const uint8_t* A, const uint8_t* B, int64_t M, int64_t N, int64_t K, int64_t b_rows,
+                     int64_t lda, int64_t ldb, float out_scale, void* C, int64_t ldc, void* stream);
+int dopt_fp8_gemm_kn_preferred(int64_t M, int64_t N, int64_t K);
+
+/*
  * Layout conversion for dopt_fp8_gemm_nt: dst[r * ld_dst + c] = src[r * stride_r + c * stride_c]
  * (byte matrices, element strides in bytes). The reference's Triton_Linear
  * (Activation_Compression/triton_kernel/linear.py:43-95) takes A [M, K] and B [K, N] with arbitrary

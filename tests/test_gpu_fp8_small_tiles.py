@@ -61,6 +61,43 @@ def test_tile_edges(M, N, K, padded):
     assert torch.equal(c, first)  # the split K is summed in a fixed order
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 16, 1), (17, 48, 100), (33, 64, 128), (64, 80, 513), (129, 144, 640), (985, 768, 1536),
+                                   (300, 1040, 1111), (1000, 2064, 400), (2050, 3088, 272)])
+@pytest.mark.parametrize("padded", [False, True])
+def test_row_major_b(M, N, K, padded):
+    """B in [K, N] rows, at the edges of every tile and of the slabs, with 0 to 15 rows less than A's padded K and
+    with rows whose padding (and the memory after the last row) holds NaN; fp8_linear gives the same bits where it
+    takes this way."""
+    gen = torch.Generator(device=DEV).manual_seed(M + 5 * N + K)
+    kp, ldb = (K + 15) // 16 * 16, N + 32 * padded
+    a = torch.zeros((M, kp), device=DEV).to(torch.float8_e4m3fn)
+    a[:, :K] = fp8((M, K), gen)
+    store = torch.full(((K + 20) * ldb,), NAN8, dtype=torch.uint8, device=DEV).view(torch.float8_e4m3fn)
+    b = store[: K * ldb].view(K, ldb)
+    b[:, :N] = fp8((K, N), gen)
+    c = torch.full((M + 1, N + 3 * padded), 55.0, dtype=torch.bfloat16, device=DEV)
+    st = torch.cuda.current_stream().cuda_stream
+    rc = _lib.lib().dopt_fp8_gemm_kn(a.data_ptr(), b.data_ptr(), M, N, kp, K, kp, ldb, 0.125, c.data_ptr(), c.shape[1], st)
+    _lib.check(rc, "fp8_gemm_kn")
+    check(c[:M, :N], a[:, :K], b[:, :N].t(), 0.125)
+    assert bool((c[:M, N:] == 55.0).all()) and bool((c[M:] == 55.0).all())
+    got = torch.ops.act_lib.fp8_linear(a[:, :K], b[:, :N], 0.125)
+    if _lib.lib().dopt_fp8_gemm_kn_preferred(M, N, kp):
+        assert torch.equal(got, c[:M, :N])
+
+
+def test_row_major_b_refuses():
+    a, b = (torch.zeros(4096, dtype=torch.uint8, device=DEV) for _ in range(2))
+    c = torch.zeros((16, 32), dtype=torch.bfloat16, device=DEV)
+    call = _lib.lib().dopt_fp8_gemm_kn
+    ok = dict(M=16, N=32, K=32, rows=32, lda=32, ldb=32, ldc=32, at=b.data_ptr())
+    for bad in (dict(N=24), dict(K=24, rows=24), dict(rows=16), dict(rows=33), dict(lda=16), dict(ldb=16), dict(ldb=40),
+                dict(ldc=16), dict(at=b.data_ptr() + 8), dict(ldb=1 << 23)):
+        v = {**ok, **bad}
+        assert call(a.data_ptr(), v["at"], v["M"], v["N"], v["K"], v["rows"], v["lda"], v["ldb"], 1.0, c.data_ptr(),
+                    v["ldc"], torch.cuda.current_stream().cuda_stream) in (_lib.EINVAL, _lib.EUNSUPPORTED), bad
+
+
 @pytest.mark.parametrize("rows,cols", [(1, 1), (16, 16), (127, 129), (128, 128), (130, 127), (1000, 77), (513, 300)])
 @pytest.mark.parametrize("layout", ["transposed", "rows", "gather"])
 @pytest.mark.parametrize("shift", [0, 3])
