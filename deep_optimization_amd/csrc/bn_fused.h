@@ -77,7 +77,8 @@ struct BnBwdArgs {
 };
 
 // vw: elements per vector access (8, 4, 2 or 1); it divides HW, stride_n and stride_c, and every
-// element pointer is aligned to vw elements (bn_width in the C ABI picks it)
+// element pointer is aligned to vw elements; or 0: accesses of 8 elements at any element, for
+// HW >= 8 and N * HW a multiple of 8 (bn_width in the C ABI picks it)
 int64_t bn_nchunks(int64_t M);
 // finalize = false: only the workgroup partials (for a consumer that sums them itself)
 int launch_bn_reduce(const void* x, int dt, const BnGeom& g, float* partial, float* sum, float* sumsq, int vw,

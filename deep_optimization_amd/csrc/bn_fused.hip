@@ -34,8 +34,12 @@
 // 8 per lane per block, read and written as 8 / V row-contiguous accesses of V elements, V the
 // largest of 8, 4, 2, 1 that divides HW and both strides and fits the pointers' alignment (so an
 // access never crosses a row: one 16-byte access for 2-byte types at HW = 56 x 56, two 8-byte
-// ones at 14 x 14, eight 2-byte ones at 7 x 7), with every block's loads issued before the first
-// is used. A group of G elements spans G/8 aligned lanes (4..64), so group min/max and the
+// ones at 14 x 14), with every block's loads issued before the first is used. Where V would be 2 or 1
+// (7 x 7, 13 x 13, unaligned tensors) and a row has 8 elements or more, V = 0 stands for 16-byte accesses at
+// any element (load8_rows, store8_rows): each access of a wave touches every cache line of its 1 KB whatever
+// its width, so eight 2-byte ones cost eight times the address work (bf16 [128, 2048, 7, 7], squashed, us:
+// statistics 25.5 -> 12.1, forward 54.7 -> 26.0, reduce 27.0 -> 12.8, dx 50.2 -> 21.8; with the channel order of
+// channel_of 10.6, 24.4, 12.4, 19.1). A group of G elements spans G/8 aligned lanes (4..64), so group min/max and the
 // code merge stay inside a wave. Reductions are two-stage and ordered (workgroup partials, then
 // one wave per channel), so sums are deterministic and need no zeroed buffer or atomics.
 #include "bn_fused.h"
@@ -73,6 +77,17 @@ __device__ __forceinline__ void cursor_step(RowCursor& p, const BnGeom& g, uint3
         p.r -= (uint32_t)g.HW;
         p.row += g.stride_n;
     }
+}
+
+// The channel of a workgroup. Short rows (V below 8) share their first and last cache lines with the neighbouring
+// channels' rows: consecutive workgroups go to the 8 XCDs in turn, so XCD k takes the k-th eighth of the channels
+// and a line is read, and its two parts are merged on writing, in one L2 (bf16, the four kernels: [128, 2048, 7, 7]
+// 74.2 -> 67.9 us, [64, 1024, 14, 14] 60.9 -> 57.6 us; no difference for whole lines).
+template <int V>
+__device__ __forceinline__ int64_t channel_of() {
+    const uint32_t x = blockIdx.x, C = gridDim.x;
+    if (V == EPL || C % 8) return x;
+    return (x % 8) * (C / 8) + x / 8;
 }
 
 // the chunk of a workgroup of the kernels that walk a channel last chunk first (see the grid above)
@@ -137,11 +152,112 @@ __device__ __forceinline__ void ldv(const void* base, int64_t off, float* v) {
     }
 }
 
-// the lane's 8 elements e0..e0+7 (cursor p at e0) as EPL / V row-contiguous loads; chunks at or
-// past M read as 0 (M is a multiple of V, so a chunk is all in or all out)
+// c ? a : b of values (a conditional expression of two array elements selects their address, and the array then
+// lives in memory)
+__device__ __forceinline__ uint32_t pick(bool c, uint32_t a, uint32_t b) { return c ? a : b; }
+
+// 16 bytes at any address a multiple of the element size (hardware takes unaligned global accesses)
+__device__ __forceinline__ uint4 ld16_any(const char* p) {
+    uint4 u;
+    __builtin_memcpy(&u, p, 16);
+    return u;
+}
+__device__ __forceinline__ void st16_any(uint16_t* p, const uint4& u) { __builtin_memcpy(p, &u, 16); }
+
+// The lane's 8 elements at cursor p where HW is at least 8 and neither row nor tensor need be aligned: the 8
+// elements from r0 = min(r, HW - 8) of the row, the first 8 of the next row if s = r - r0 of the lane's lie there
+// (else the same again), and the 8 elements from s on of the two together, so every load stays in its row.
+template <int DT>
+__device__ __forceinline__ void load8_rows(const void* base, const BnGeom& g, const RowCursor& p, float* v) {
+    constexpr int B = DType<DT>::bytes, D = 2 * B;  // dwords of 8 elements
+    const uint32_t r0 = min(p.r, (uint32_t)g.HW - 8u), s = p.r - r0;
+    const char* pa = (const char*)base + (p.row + r0) * B;
+    const char* pb = s ? (const char*)base + (p.row + g.stride_n) * B : pa;
+    uint32_t w[2 * D];
+#pragma unroll
+    for (int h = 0; h < D / 4; ++h) {
+        const uint4 a = ld16_any(pa + 16 * h), b = ld16_any(pb + 16 * h);
+        w[4 * h] = a.x; w[4 * h + 1] = a.y; w[4 * h + 2] = a.z; w[4 * h + 3] = a.w;
+        w[D + 4 * h] = b.x; w[D + 4 * h + 1] = b.y; w[D + 4 * h + 2] = b.z; w[D + 4 * h + 3] = b.w;
+    }
+    // shift left by s elements: 4, then 2, then 1
+    const bool s4 = s & 4u, s2 = s & 2u, s1 = s & 1u;
+#pragma unroll
+    for (int i = 0; i + D / 2 < 2 * D; ++i) w[i] = pick(s4, w[i + D / 2], w[i]);
+#pragma unroll
+    for (int i = 0; i < D + D / 8 + (D == 8 ? 0 : 1); ++i) w[i] = pick(s2, w[i + D / 4], w[i]);
+    if constexpr (B == 4) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = __uint_as_float(pick(s1, w[i + 1], w[i]));
+    } else {
+        uint4 u;
+        u.x = __builtin_amdgcn_alignbit(w[1], w[0], s1 ? 16u : 0u);
+        u.y = __builtin_amdgcn_alignbit(w[2], w[1], s1 ? 16u : 0u);
+        u.z = __builtin_amdgcn_alignbit(w[3], w[2], s1 ? 16u : 0u);
+        u.w = __builtin_amdgcn_alignbit(w[4], w[3], s1 ? 16u : 0u);
+        widen16<DT>(u, v);
+    }
+}
+
+// the 8 bf16 values that end s (0..7) elements before the end of the 16 in (a, b)
+__device__ __forceinline__ uint4 window8(const uint32_t* a, const uint32_t* b, uint32_t s) {
+    uint32_t w[8], t[6], u[5], o[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        w[i] = a[i];
+        w[4 + i] = b[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 6; ++i) t[i] = pick(s & 4u, w[i], w[i + 2]);
+#pragma unroll
+    for (int i = 0; i < 5; ++i) u[i] = pick(s & 2u, t[i], t[i + 1]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = pick(s & 1u, __builtin_amdgcn_alignbit(u[i + 1], u[i], 16u), u[i + 1]);
+    return make_uint4(o[0], o[1], o[2], o[3]);
+}
+
+// Writes the lane's 8 values where load8_rows reads them. A lane whose values run into the next row (s of them)
+// writes the last 8 elements of the one row and the first 8 of the other, with its neighbours' values (the wave
+// holds 512 consecutive elements) beside its own; both lanes of an overlap write the same bytes. The wave's first
+// and last lane have no such neighbour and write their part of a crossed row by element. (A crossing lane's
+// neighbours are active: they lie below M as its own elements do, on both sides in the same rows.)
+__device__ __forceinline__ void store8_rows(uint16_t* base, const BnGeom& g, const RowCursor& p, const float* v) {
+    const uint32_t d[4] = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7])};
+    const uint32_t r0 = min(p.r, (uint32_t)g.HW - 8u), s = p.r - r0;
+    uint32_t prev[4], next[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        prev[i] = dpp_u32<0x138>(d[i]);  // wave_shr:1, lane - 1's
+        next[i] = dpp_u32<0x130>(d[i]);  // wave_shl:1, lane + 1's
+    }
+    const int lane = threadIdx.x & 63;
+    uint16_t* q = base + p.row;
+    uint16_t* q2 = q + g.stride_n;
+    if (s == 0 || lane != 0) {
+        st16_any(q + r0, window8(prev, d, s));
+    } else {
+#pragma unroll
+        for (int k = 0; k < 7; ++k)
+            if (k < 8 - (int)s) q[p.r + k] = (uint16_t)(d[k >> 1] >> (16 * (k & 1)));
+    }
+    if (s) {
+        if (lane != 63) {
+            st16_any(q2, window8(d, next, s));
+        } else {
+#pragma unroll
+            for (int k = 1; k < 8; ++k)
+                if (k >= 8 - (int)s) q2[k - 8 + (int)s] = (uint16_t)(d[k >> 1] >> (16 * (k & 1)));
+        }
+    }
+}
+
+// the lane's 8 elements e0..e0+7 (cursor p at e0) as EPL / V row-contiguous loads (or load8_rows at V = 0);
+// chunks at or past M read as 0 (M is a multiple of V, so a chunk is all in or all out)
 template <int DT, int V>
 __device__ __forceinline__ void load8(const void* base, const BnGeom& g, RowCursor p, int64_t e0, int64_t M,
                                       float* v) {
+    if constexpr (V == 0) return load8_rows<DT>(base, g, p, v);  // M % 8 == 0: e0 < M for every caller
+    else
 #pragma unroll
     for (int j = 0; j < EPL / V; ++j) {
         if (j) cursor_step(p, g, V, 0);
@@ -158,6 +274,8 @@ __device__ __forceinline__ void load8(const void* base, const BnGeom& g, RowCurs
 template <int V>
 __device__ __forceinline__ void store8_bf16(uint16_t* base, const BnGeom& g, RowCursor p, int64_t e0, int64_t M,
                                             const float* v) {
+    if constexpr (V == 0) return store8_rows(base, g, p, v);
+    else
 #pragma unroll
     for (int j = 0; j < EPL / V; ++j) {
         if (j) cursor_step(p, g, V, 0);
@@ -303,7 +421,7 @@ __device__ __forceinline__ void lane_codes(const BnBwdArgs& a, int64_t c, int64_
 template <int DT, int V>
 __global__ __launch_bounds__(TPB) void bn_stats_kernel(const void* __restrict__ x, BnGeom g,
                                                        float* __restrict__ partial, int64_t nchunks) {
-    const int64_t c = blockIdx.x, chunk = blockIdx.y;
+    const int64_t c = channel_of<V>(), chunk = blockIdx.y;
     const int64_t M = g.N * g.HW;
     const int64_t base = chunk * BN_CHUNK + (int64_t)threadIdx.x * EPL;
     RowCursor cur[ITER];
@@ -580,7 +698,7 @@ __device__ __forceinline__ void fwd_block(const BnFwdArgs& a, int64_t c, RowCurs
 // before the first block is processed.
 template <int DT, int MODE, int V, bool R6, bool ALAM = false, bool THR = false>
 __global__ __launch_bounds__(TPB) void bn_fwd_kernel(BnFwdArgs a, int lg, int bits) {
-    const int64_t c = blockIdx.x;
+    const int64_t c = channel_of<V>();
     const int64_t M = a.g.N * a.g.HW;
     const int64_t base = reversed_chunk() * BN_CHUNK + (int64_t)threadIdx.x * EPL;
     RowCursor cur[ITER];
@@ -664,7 +782,7 @@ __device__ __forceinline__ void bwd_codes(const BnBwdArgs& a, int64_t c, RowCurs
 // index of the reference's two-group block; the seed does not depend on the channel.
 template <int DYT, int MODE, int V, bool ALAM = false>
 __global__ __launch_bounds__(TPB) void bn_bwd_reduce_kernel(BnBwdArgs a, int lg, int bits, int64_t nchunks) {
-    const int64_t c = blockIdx.x, chunk = blockIdx.y;
+    const int64_t c = channel_of<V>(), chunk = blockIdx.y;
     const int64_t M = a.g.N * a.g.HW;
     const int64_t base = chunk * BN_CHUNK + (int64_t)threadIdx.x * EPL;
     RowCursor cur[ITER];
@@ -736,7 +854,7 @@ __global__ __launch_bounds__(TPB) void bn_bwd_reduce_kernel(BnBwdArgs a, int lg,
 
 template <int DYT, int MODE, int V, bool ALAM = false>
 __global__ __launch_bounds__(TPB) void bn_bwd_dx_kernel(BnBwdArgs a, int lg, int bits) {
-    const int64_t c = blockIdx.x;
+    const int64_t c = channel_of<V>();
     const int64_t M = a.g.N * a.g.HW;
     const int64_t base = reversed_chunk() * BN_CHUNK + (int64_t)threadIdx.x * EPL;
     RowCursor cur[ITER];
@@ -783,13 +901,14 @@ int log2i(int v) {
     return l;
 }
 
-// kernel template for the vector width vw (8, 4, 2 or 1 elements per access)
+// kernel template for the vector width vw (8, 4, 2 or 1 elements per access, or 0: 8 at any element)
 #define DOPT_BN_BY_WIDTH(vw, LAUNCH) \
     do {                             \
         switch (vw) {                \
             case 8: LAUNCH(8); break; \
             case 4: LAUNCH(4); break; \
             case 2: LAUNCH(2); break; \
+            case 0: LAUNCH(0); break; \
             default: LAUNCH(1); break; \
         }                            \
     } while (0)

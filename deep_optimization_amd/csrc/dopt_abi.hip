@@ -122,6 +122,7 @@ struct BnTensor {
 };
 int bn_width(const dopt::BnGeom& g, std::initializer_list<BnTensor> ts) {
     for (int v : {8, 4, 2}) {
+        if (v == 2 && g.HW >= 8 && g.N * g.HW % 8 == 0) return 0;  // faster than 2 or 1 element at a time (bn_fused.hip)
         if (g.HW % v || g.stride_n % v || g.stride_c % v) continue;
         bool ok = true;
         for (const BnTensor& t : ts) {

@@ -577,3 +577,42 @@ def test_alam_operator_opcheck():
     dw, db = ops.bn_bwd_reduce_dequant_unpack_fused(packed, dy, scale, mn, **bk)
     torch.library.opcheck(ops.bn_bwd_dx_dequant_unpack_fused.default, (packed, dy, scale, mn, dw, db, w.to(DEV), var),
                           dict(bk, sync=False), test_utils=tests)
+
+
+# rows of 8 elements or more that no 8-byte access fits (every kernel's 16-byte accesses at any element), a row of 8
+# (each of the 8 positions of a crossing), rows shorter than a lane's 8 elements, unaligned tensors with wide rows,
+# and channel counts that are and are not a multiple of 8
+ROWS = [(32, 8, 7 * 7), (64, 5, 9), (32, 16, 10), (32, 3, 169), (96, 8, 11), (32, 8, 15), (160, 2, 13), (64, 8, 5), (33, 8, 32),
+        (4, 8, 256)]
+
+
+@pytest.mark.parametrize("N,C,HW", ROWS)
+@pytest.mark.parametrize("dtype", DTYPES, ids=["bf16", "f32", "f16"])
+@pytest.mark.parametrize("kind,bits", [(1, 2), (1, 4), (2, 2), (3, 8)])
+@pytest.mark.parametrize("shift", [0, 1, 3])
+def test_short_and_unaligned_rows(N, C, HW, dtype, kind, bits, shift):
+    """The layer operators on [N, C, HW] equal, bit for bit, the same channels as one aligned row each ([1, C, N * HW]:
+    8 elements per access), with x and dy at an element offset."""
+    if shift == 0 and HW % 4 == 0:
+        pytest.skip("aligned wide rows: covered above")
+    gen = torch.Generator(device=DEV).manual_seed(N + HW + bits)
+
+    def rows(t):  # [N, C, HW] -> [1, C, N * HW]
+        return t.view(N, C, HW).transpose(0, 1).reshape(1, C, N * HW).contiguous()
+
+    def tensor(dt):
+        t = torch.randn(N * C * HW + shift, generator=gen, device=DEV).to(dt)
+        return t[shift:].view(N, C, HW)
+
+    x, dy = tensor(dtype), tensor(dtype)
+    w, b = torch.rand(C, generator=gen, device=DEV) + 0.5, torch.randn(C, generator=gen, device=DEV)
+    out = []
+    for X, DY in ((x, dy), (rows(x), rows(dy))):
+        rm, rv = torch.zeros(C, device=DEV), torch.ones(C, device=DEV)
+        y, packed, rp, scale, xmin, mean, var = ops.bn_train_fwd(X, w, b, rm, rv, 0.1, 64, bits, kind)
+        dx, dw, db = ops.bn_train_bwd(packed, rp if kind != 1 else None, DY, scale, xmin, w, var, 64, bits, kind)
+        out.append((y.view(X.shape), packed, scale, xmin, rp, mean, var, rm, rv, dx.view(X.shape), dw, db))
+    for i, (got, want) in enumerate(zip(*out)):
+        if i in (0, 9):
+            got = rows(got)
+        assert torch.equal(got.view(torch.uint8), want.view(torch.uint8)), i
