@@ -213,7 +213,7 @@ __global__ __launch_bounds__(256, 1) void fp8_gemm_mid_kernel(Fp8GemmArgs p) {
     __syncthreads();
 
     // epilogue: scale, round once, stage the wave's WM x WN bf16 tile in an LDS array of its own, write
-    // 16-byte row chunks (element stores for a ragged last chunk or an unaligned C)
+    // 16-byte row chunks (element stores for a ragged last chunk)
     constexpr int PITCH = WN + 8;  // bf16 per staged row
     static_assert(WM * PITCH * 2 <= BM * BK, "a wave's tile fits one LDS array");
     uint16_t* tile = (uint16_t*)(wave == 0 ? sA0 : wave == 1 ? sA1 : wave == 2 ? sA2 : sA3);
@@ -235,8 +235,8 @@ __global__ __launch_bounds__(256, 1) void fp8_gemm_mid_kernel(Fp8GemmArgs p) {
         if (m >= M || n >= N) continue;
         uint16_t* dst = p.C + m * ldc + n;
         const uint16_t* src = tile + r * PITCH + c;
-        if (p.vec_store && n + 8 <= N) {
-            *(v4u_t*)dst = *(const v4u_t*)src;
+        if (n + 8 <= N) {
+            store_c8(dst, *(const v4u_t*)src);
         } else {
 #pragma unroll 1
             for (int e = 0; e < 8 && n + e < N; ++e) dst[e] = src[e];

@@ -122,8 +122,8 @@ __global__ __launch_bounds__(64 * NW) void fp8_gemm_small_kernel(Fp8GemmArgs p) 
                          pack_bf16x2(s1[0] * p.out_scale, s1[1] * p.out_scale),
                          pack_bf16x2(s1[2] * p.out_scale, s1[3] * p.out_scale)};
         uint16_t* dst = p.C + m * ldc + n;
-        if (p.vec_store && n + 8 <= N) {
-            *(v4u_t*)dst = v;
+        if (n + 8 <= N) {
+            store_c8(dst, v);
         } else {
             const uint16_t e8[8] = {(uint16_t)v.x, (uint16_t)(v.x >> 16), (uint16_t)v.y, (uint16_t)(v.y >> 16),
                                     (uint16_t)v.z, (uint16_t)(v.z >> 16), (uint16_t)v.w, (uint16_t)(v.w >> 16)};
