@@ -31,6 +31,7 @@ EXPORTS = (
     "dopt_fp8_gemm_kn",
     "dopt_fp8_gemm_kn_preferred",
     "dopt_fp8_pack_kmajor",
+    "dopt_fp8_pack_kmajor_padded",
     "dopt_relu_pack",
     "dopt_relu_unpack",
     "dopt_act_forward",
@@ -100,6 +101,8 @@ def lib() -> ctypes.CDLL:
         L.dopt_fp8_gemm_kn_preferred.restype = i32
         L.dopt_fp8_pack_kmajor.argtypes = [vp, i64, i64, i64, i64, vp, i64, vp]
         L.dopt_fp8_pack_kmajor.restype = i32
+        L.dopt_fp8_pack_kmajor_padded.argtypes = [vp, i64, i64, i64, i64, vp, i64, i64, vp]
+        L.dopt_fp8_pack_kmajor_padded.restype = i32
         L.dopt_relu_pack.argtypes = [vp, i32, i64, i32, i32, vp, vp, vp]
         L.dopt_relu_pack.restype = i32
         L.dopt_relu_unpack.argtypes = [vp, vp, i32, i64, i32, vp, vp]

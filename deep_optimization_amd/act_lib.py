@@ -434,11 +434,12 @@ fp8_gemm_nt = _op(
 def _kmajor(t: Tensor, rows: int, k: int, stride_r: int, stride_k: int, k_pad: int):
     """(tensor, row stride) of an e4m3 operand as the GEMM reads it: rows K-contiguous, row stride a
     multiple of 16, 16-byte aligned. Used in place when it already is; otherwise packed by
-    dopt_fp8_pack_kmajor into a fresh [rows, k_pad] buffer whose padding columns are zero."""
+    dopt_fp8_pack_kmajor_padded into a fresh [rows, k_pad] buffer whose padding columns are zero."""
     if stride_k == 1 and k == k_pad and stride_r % 16 == 0 and k <= stride_r < (1 << 23) and t.data_ptr() % 16 == 0:
         return t, stride_r
-    out = (torch.zeros if k_pad != k else torch.empty)((rows, k_pad), dtype=torch.uint8, device=t.device)
-    rc = _lib.lib().dopt_fp8_pack_kmajor(t.data_ptr(), rows, k, stride_r, stride_k, out.data_ptr(), k_pad, _stream(t))
+    out = torch.empty((rows, k_pad), dtype=torch.uint8, device=t.device)
+    rc = _lib.lib().dopt_fp8_pack_kmajor_padded(t.data_ptr(), rows, k, stride_r, stride_k, out.data_ptr(), k_pad, k_pad,
+                                                _stream(t))
     _lib.check(rc, "fp8_pack_kmajor")
     return out, k_pad
 
@@ -448,8 +449,8 @@ def _fp8_linear(a, b, out_scale):
     a [M, K] @ b [K, N] with any strides -> bf16 [M, N] = out_scale * a @ b, fp32 accumulate. The
     GEMM reads both operands K-contiguous: an operand in another layout (b in its row-major [K, N]
     layout, a transposed view, unaligned rows, K not a multiple of 16) is first packed by
-    dopt_fp8_pack_kmajor (zero-padding K to a multiple of 16), the rest is read in place. A row-major b
-    with 16-byte rows is read as it lies where that is the faster way (dopt_fp8_gemm_kn)."""
+    dopt_fp8_pack_kmajor_padded (zero-padding K to a multiple of 16), the rest is read in place. A row-major b
+    is read as it lies, or from a copy with 16-byte rows, where that is the faster way (dopt_fp8_gemm_kn)."""
     if a.dtype != torch.float8_e4m3fn or b.dtype != torch.float8_e4m3fn:
         raise RuntimeError("fp8_linear expects torch.float8_e4m3fn operands")
     if a.dim() != 2 or b.dim() != 2 or a.shape[1] != b.shape[0]:
@@ -464,10 +465,15 @@ def _fp8_linear(a, b, out_scale):
         return c.zero_()
     k_pad = (K + 15) // 16 * 16
     ta, lda = _kmajor(a.view(torch.uint8), M, K, a.stride(0), a.stride(1), k_pad)
-    ldb = b.stride(0)
-    if b.stride(1) == 1 and ldb % 16 == 0 and N <= ldb < (1 << 23) and N % 16 == 0 and b.data_ptr() % 16 == 0 and \
-            _lib.lib().dopt_fp8_gemm_kn_preferred(M, N, k_pad):
-        rc = _lib.lib().dopt_fp8_gemm_kn(ta.data_ptr(), b.data_ptr(), M, N, k_pad, K, lda, ldb, float(out_scale),
+    if b.stride(1) == 1 and _lib.lib().dopt_fp8_gemm_kn_preferred(M, N, k_pad):
+        tb, ldb = b.view(torch.uint8), b.stride(0)
+        if ldb % 16 or not N <= ldb < (1 << 23) or N % 16 or b.data_ptr() % 16:  # a copy with aligned rows
+            ldb = (N + 15) // 16 * 16
+            tb = torch.empty((K, ldb), dtype=torch.uint8, device=a.device)
+            rc = _lib.lib().dopt_fp8_pack_kmajor_padded(b.data_ptr(), K, N, b.stride(0), 1, tb.data_ptr(), ldb, ldb,
+                                                        _stream(a))
+            _lib.check(rc, "fp8_pack_kmajor")
+        rc = _lib.lib().dopt_fp8_gemm_kn(ta.data_ptr(), tb.data_ptr(), M, N, k_pad, K, lda, ldb, float(out_scale),
                                          c.data_ptr(), N, _stream(a))
         _lib.check(rc, "fp8_linear")
         return c

@@ -21,7 +21,7 @@ int launch_fp8_gemm_kn(const uint8_t* A, const uint8_t* B, int64_t M, int64_t N,
                        int64_t ldb, float out_scale, uint16_t* C, int64_t ldc, hipStream_t s);
 bool fp8_gemm_kn_preferred(int64_t M, int64_t N, int64_t K);
 int launch_fp8_pack(const uint8_t* src, int64_t rows, int64_t cols, int64_t stride_r, int64_t stride_c, uint8_t* dst,
-                    int64_t ld_dst, hipStream_t s);
+                    int64_t ld_dst, int64_t cols_out, hipStream_t s);
 int launch_relu_pack(const void* x, int dt, void* y, uint32_t* packed, uint64_t n, int bits, bool relu6, hipStream_t s);
 int launch_relu_unpack(const uint32_t* packed, const void* dy, int dyt, void* dx, uint64_t n, int bits, hipStream_t s);
 int launch_act_forward(const void* x, int dt, void* y, void* aux, uint64_t n, int act, hipStream_t s);
@@ -414,15 +414,14 @@ int dopt_fp8_gemm_kn(const uint8_t* A, const uint8_t* B, int64_t M, int64_t N, i
     if (M < 0 || N < 0 || K < 0) return fail(DOPT_EINVAL, "negative GEMM extent");
     if (M == 0 || N == 0) return ok();
     if (K == 0 || !A || !B || !C) return fail(DOPT_EINVAL, "fp8_gemm_kn: K is 0 or a pointer is null");
-    if (K % 16 || N % 16)
-        return fail(DOPT_EUNSUPPORTED, "fp8_gemm_kn needs K %% 16 == 0 and N %% 16 == 0, got K=%lld N=%lld", (long long)K,
-                    (long long)N);
+    if (K % 16)
+        return fail(DOPT_EUNSUPPORTED, "fp8_gemm_kn needs K %% 16 == 0, got K=%lld", (long long)K);
     if (b_rows > K || b_rows <= K - 16)
         return fail(DOPT_EINVAL, "fp8_gemm_kn: B has K rows or up to 15 fewer, got %lld of %lld", (long long)b_rows,
                     (long long)K);
     if (lda < K || ldb < N || ldc < N || lda % 16 || ldb % 16 || !aligned16(A) || !aligned16(B) || ((uintptr_t)C & 1))
         return fail(DOPT_EINVAL,
-                    "fp8_gemm_kn needs 16-byte aligned A and B, lda >= K and ldb >= N multiples of 16, a 2-byte aligned C "
+                    "fp8_gemm_kn needs 16-byte aligned A and B, multiples of 16 lda >= K and ldb >= N, a 2-byte aligned C "
                     "and ldc >= N (got lda=%lld ldb=%lld ldc=%lld K=%lld N=%lld)",
                     (long long)lda, (long long)ldb, (long long)ldc, (long long)K, (long long)N);
     if (lda >= (1 << 23) || ldb >= (1 << 23))
@@ -437,13 +436,21 @@ int dopt_fp8_gemm_kn(const uint8_t* A, const uint8_t* B, int64_t M, int64_t N, i
 
 int dopt_fp8_pack_kmajor(const uint8_t* src, int64_t rows, int64_t cols, int64_t stride_r, int64_t stride_c, uint8_t* dst,
                          int64_t ld_dst, void* stream) {
+    return dopt_fp8_pack_kmajor_padded(src, rows, cols, stride_r, stride_c, dst, ld_dst, cols, stream);
+}
+
+int dopt_fp8_pack_kmajor_padded(const uint8_t* src, int64_t rows, int64_t cols, int64_t stride_r, int64_t stride_c,
+                                uint8_t* dst, int64_t ld_dst, int64_t cols_out, void* stream) {
     if (rows < 0 || cols < 0 || stride_r < 0 || stride_c < 0)
         return fail(DOPT_EINVAL, "fp8 pack: negative extent or stride");
     if (rows == 0 || cols == 0) return ok();
     if (!src || !dst) return fail(DOPT_EINVAL, "null pointer argument");
     if (ld_dst < cols) return fail(DOPT_EINVAL, "fp8 pack: ld_dst (%lld) < cols (%lld)", (long long)ld_dst, (long long)cols);
+    if (cols_out < cols || cols_out > ld_dst || cols_out - cols > 15)
+        return fail(DOPT_EINVAL, "fp8 pack: %lld columns out of %lld: at most 15 more, and within ld_dst (%lld)",
+                    (long long)cols_out, (long long)cols, (long long)ld_dst);
     (void)hipGetLastError();
-    if (dopt::launch_fp8_pack(src, rows, cols, stride_r, stride_c, dst, ld_dst, (hipStream_t)stream))
+    if (dopt::launch_fp8_pack(src, rows, cols, stride_r, stride_c, dst, ld_dst, cols_out, (hipStream_t)stream))
         return fail(DOPT_EINVAL, "fp8 pack: %lld x %lld is too large for one launch", (long long)rows, (long long)cols);
     return hip_status("fp8_pack launch");
 }

@@ -14,7 +14,8 @@
 // LDS rows are the slab's 128 bytes; 16-byte chunk c of row r lies at c ^ f(r), f as in
 // fp8_gemm16_persistent_kernel (the same 16-row fragments).
 //
-// KN: B lies as [K, N] rows (a weight used as x @ w), N and its row stride multiples of 16 bytes. Its slab is
+// KN: B lies as [K, N] rows (a weight used as x @ w) at a stride of a multiple of 16 bytes, each row readable up to
+// N rounded up to one (the bytes past N only reach columns that are not stored). Its slab is
 // then 128 rows of BN bytes, loaded as they lie, and the operand reads transpose: ds_read_b64_tr_b8 hands 16
 // lanes an 8 x 16 block of bytes by columns, four of them make a fragment's 32 K bytes per lane (the K order of
 // the other form, so the sums are the same bit for bit). 16-byte chunk c of row k lies at c ^ g(k), so the 16
@@ -106,7 +107,7 @@ __global__ __launch_bounds__(256, 1) void fp8_gemm_mid_kernel(Fp8GemmArgs p) {
         if constexpr (KN) {
             // the slab's rows end with B's last: the buffer range covers what is left of it, so rows past it
             // read zeros (a slab's offsets stay below 2^30, so a range cut to GEMM_RANGE covers whole slabs)
-            const int64_t left = (p.b_rows - 1 - (int64_t)k0) * ldb + N - n0;
+            const int64_t left = (p.b_rows - 1 - (int64_t)k0) * ldb + (N + 15) / 16 * 16 - n0;
             const int range = left <= 0 ? 0 : left < (int64_t)GEMM_RANGE ? (int)left : (int)GEMM_RANGE;
             const __amdgpu_buffer_rsrc_t rk =
                 __builtin_amdgcn_make_buffer_rsrc((void*)(p.B + (int64_t)k0 * ldb + n0), (short)0, range, 0x00020000);

@@ -484,9 +484,9 @@ std::pair<Tensor, int64_t> kmajor(const Tensor& t, int64_t rows, int64_t k, int6
         reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0)
         return {t, stride_r};
     const auto bytes = t.options().dtype(at::kByte);
-    Tensor out = k_pad != k ? at::zeros({rows, k_pad}, bytes) : at::empty({rows, k_pad}, bytes);
-    check(dopt_fp8_pack_kmajor((const uint8_t*)t.data_ptr(), rows, k, stride_r, stride_k, (uint8_t*)out.data_ptr(), k_pad,
-                               stream_of(t)),
+    Tensor out = at::empty({rows, k_pad}, bytes);
+    check(dopt_fp8_pack_kmajor_padded((const uint8_t*)t.data_ptr(), rows, k, stride_r, stride_k, (uint8_t*)out.data_ptr(),
+                                      k_pad, k_pad, stream_of(t)),
           "fp8_pack_kmajor");
     return {out, k_pad};
 }
@@ -505,9 +505,17 @@ Tensor fp8_linear(const Tensor& a, const Tensor& b, double out_scale) {
     if (K == 0) return c.zero_();
     const int64_t k_pad = (K + 15) / 16 * 16;
     const auto [ta, lda] = kmajor(a, M, K, a.stride(0), a.stride(1), k_pad);
-    if (b.stride(1) == 1 && N % 16 == 0 && b.stride(0) % 16 == 0 && N <= b.stride(0) && b.stride(0) < (1 << 23) &&
-        reinterpret_cast<uintptr_t>(b.data_ptr()) % 16 == 0 && dopt_fp8_gemm_kn_preferred(M, N, k_pad)) {
-        check(dopt_fp8_gemm_kn((const uint8_t*)ta.data_ptr(), (const uint8_t*)b.data_ptr(), M, N, k_pad, K, lda, b.stride(0),
+    if (b.stride(1) == 1 && dopt_fp8_gemm_kn_preferred(M, N, k_pad)) {
+        Tensor tb = b;
+        int64_t ldb = b.stride(0);
+        if (ldb % 16 || ldb < N || ldb >= (1 << 23) || N % 16 || reinterpret_cast<uintptr_t>(b.data_ptr()) % 16) {
+            ldb = (N + 15) / 16 * 16;  // a copy with aligned rows
+            tb = at::empty({K, ldb}, b.options().dtype(at::kByte));
+            check(dopt_fp8_pack_kmajor_padded((const uint8_t*)b.data_ptr(), K, N, b.stride(0), 1, (uint8_t*)tb.data_ptr(),
+                                              ldb, ldb, stream_of(a)),
+                  "fp8_pack_kmajor");
+        }
+        check(dopt_fp8_gemm_kn((const uint8_t*)ta.data_ptr(), (const uint8_t*)tb.data_ptr(), M, N, k_pad, K, lda, ldb,
                                (float)out_scale, c.data_ptr(), N, stream_of(a)),
               "fp8_linear");
         return c;

@@ -154,8 +154,9 @@ int dopt_fp8_gemm_nt(const uint8_t* A, const uint8_t* B, int64_t M, int64_t N, i
 
 /*
  * The same product with B in row-major [K, N] rows (Triton_Linear's own layout), read as it lies:
- * C[m][n] = bf16(out_scale * sum_k A[m][k] * B[k][n]). N % 16 == 0 and K % 16 == 0; B may have
- * b_rows = K - 15 .. K rows (rows from b_rows to K count as zeros: A is then a copy padded to K columns).
+ * C[m][n] = bf16(out_scale * sum_k A[m][k] * B[k][n]). K % 16 == 0; B may have
+ * b_rows = K - 15 .. K rows (rows from b_rows to K count as zeros: A is then a copy padded to K columns),
+ * each readable up to N rounded up to a multiple of 16 (what lies past N is not used).
  * lda >= K and ldb >= N multiples of 16 and < 2^23, A and B 16-byte aligned, C as above.
  * dopt_fp8_gemm_kn_preferred: 1 where this is estimated to be faster than packing B for
  * dopt_fp8_gemm_nt first (outputs below the sizes that the 256 x 256 tiles need).
@@ -174,6 +175,9 @@ int dopt_fp8_gemm_kn_preferred(int64_t M, int64_t N, int64_t K);
  */
 int dopt_fp8_pack_kmajor(const uint8_t* src, int64_t rows, int64_t cols, int64_t stride_r, int64_t stride_c,
                          uint8_t* dst, int64_t ld_dst, void* stream);
+/* ... and zeros in the columns cols <= c < cols_out (at most 15 of them, cols_out <= ld_dst). */
+int dopt_fp8_pack_kmajor_padded(const uint8_t* src, int64_t rows, int64_t cols, int64_t stride_r, int64_t stride_c,
+                                uint8_t* dst, int64_t ld_dst, int64_t cols_out, void* stream);
 
 /* ---------------------------------------------------------------- fused activation layers
  * The compressed ReLU / GELU / SiLU layers of Activation_Compression/modules/activations/ save the

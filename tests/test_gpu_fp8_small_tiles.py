@@ -62,14 +62,15 @@ def test_tile_edges(M, N, K, padded):
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 16, 1), (17, 48, 100), (33, 64, 128), (64, 80, 513), (129, 144, 640), (985, 768, 1536),
-                                   (300, 1040, 1111), (1000, 2064, 400), (2050, 3088, 272)])
+                                   (300, 1040, 1111), (1000, 2064, 400), (2050, 3088, 272), (70, 33, 65), (262, 3804, 187),
+                                   (1000, 777, 1001)])
 @pytest.mark.parametrize("padded", [False, True])
 def test_row_major_b(M, N, K, padded):
     """B in [K, N] rows, at the edges of every tile and of the slabs, with 0 to 15 rows less than A's padded K and
     with rows whose padding (and the memory after the last row) holds NaN; fp8_linear gives the same bits where it
     takes this way."""
     gen = torch.Generator(device=DEV).manual_seed(M + 5 * N + K)
-    kp, ldb = (K + 15) // 16 * 16, N + 32 * padded
+    kp, ldb = (K + 15) // 16 * 16, (N + 15) // 16 * 16 + 32 * padded
     a = torch.zeros((M, kp), device=DEV).to(torch.float8_e4m3fn)
     a[:, :K] = fp8((M, K), gen)
     store = torch.full(((K + 20) * ldb,), NAN8, dtype=torch.uint8, device=DEV).view(torch.float8_e4m3fn)
@@ -91,7 +92,7 @@ def test_row_major_b_refuses():
     c = torch.zeros((16, 32), dtype=torch.bfloat16, device=DEV)
     call = _lib.lib().dopt_fp8_gemm_kn
     ok = dict(M=16, N=32, K=32, rows=32, lda=32, ldb=32, ldc=32, at=b.data_ptr())
-    for bad in (dict(N=24), dict(K=24, rows=24), dict(rows=16), dict(rows=33), dict(lda=16), dict(ldb=16), dict(ldb=40),
+    for bad in (dict(K=24, rows=24), dict(rows=16), dict(rows=33), dict(lda=16), dict(ldb=16), dict(ldb=40),
                 dict(ldc=16), dict(at=b.data_ptr() + 8), dict(ldb=1 << 23)):
         v = {**ok, **bad}
         assert call(a.data_ptr(), v["at"], v["M"], v["N"], v["K"], v["rows"], v["lda"], v["ldb"], 1.0, c.data_ptr(),
@@ -116,3 +117,10 @@ def test_pack_kmajor(rows, cols, layout, shift):
                                              ld, torch.cuda.current_stream().cuda_stream)
         _lib.check(rc, "fp8_pack_kmajor")
         assert torch.equal(dst[:, :cols], view) and bool((dst[:, cols:] == 0xAB).all())
+        for out in (cols + 3, min(cols + 15, ld)):  # and zeros in the columns up to cols_out
+            dst.fill_(0xAB)
+            rc = _lib.lib().dopt_fp8_pack_kmajor_padded(view.data_ptr(), rows, cols, view.stride(0), view.stride(1),
+                                                        dst.data_ptr(), ld, out, torch.cuda.current_stream().cuda_stream)
+            _lib.check(rc, "fp8_pack_kmajor_padded")
+            assert torch.equal(dst[:, :cols], view)
+            assert bool((dst[:, cols:out] == 0).all()) and bool((dst[:, out:] == 0xAB).all())
