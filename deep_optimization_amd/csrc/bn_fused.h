@@ -87,5 +87,9 @@ int launch_bn_fwd(const BnFwdArgs& a, int dt, int mode, int group, int bits, int
 int launch_bn_bwd_reduce(const BnBwdArgs& a, int dyt, int mode, int group, int bits, int vw, hipStream_t s,
                          bool finalize = true);
 int launch_bn_bwd_dx(const BnBwdArgs& a, int dyt, int mode, int group, int bits, int vw, hipStream_t s);
+// the statistics and normalize, or reduce and dx, of short channels in one kernel; false if the shape is not theirs.
+// Results are those of the two kernels (partials of a.nchunks chunks), bit for bit.
+bool launch_bn_fwd_whole(const BnFwdArgs& a, int dt, int mode, int group, int bits, int vw, hipStream_t s);
+bool launch_bn_bwd_whole(const BnBwdArgs& a, int dyt, int mode, int group, int bits, int vw, hipStream_t s);
 
 }  // namespace dopt

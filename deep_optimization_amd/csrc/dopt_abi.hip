@@ -745,9 +745,6 @@ int bn_train_forward_impl(bool noalloc, const void* x, int x_dtype, int64_t N, i
     if (mode == DOPT_BN_NORM && !x_hat) return fail(DOPT_EINVAL, "null x_hat pointer");
     const int vw = bn_width(g, {{x, bn_bytes(x_dtype)}, {y, 2}, {x_hat, 2}});
     (void)hipGetLastError();
-    // workgroup partials only: the normalize kernel sums them itself (no finalize launch)
-    dopt::launch_bn_reduce(x, x_dtype, g, workspace, nullptr, nullptr, bn_width(g, {{x, bn_bytes(x_dtype)}}),
-                           (hipStream_t)stream, false);
     dopt::BnFwdArgs a{};
     a.g = g;
     a.x = x;
@@ -769,7 +766,12 @@ int bn_train_forward_impl(bool noalloc, const void* x, int x_dtype, int64_t N, i
     a.run_var = running_var;
     a.run_mom = momentum;
     a.run_keep = (float)(1.0 - (double)momentum);
-    dopt::launch_bn_fwd(a, x_dtype, mode, group_size, bits, vw, (hipStream_t)stream);
+    if (!dopt::launch_bn_fwd_whole(a, x_dtype, mode, group_size, bits, vw, (hipStream_t)stream)) {
+        // workgroup partials only: the normalize kernel sums them itself (no finalize launch)
+        dopt::launch_bn_reduce(x, x_dtype, g, workspace, nullptr, nullptr, bn_width(g, {{x, bn_bytes(x_dtype)}}),
+                               (hipStream_t)stream, false);
+        dopt::launch_bn_fwd(a, x_dtype, mode, group_size, bits, vw, (hipStream_t)stream);
+    }
     return hip_status(noalloc ? "bn_train_forward_noalloc launch" : "bn_train_forward launch");
 }
 
@@ -829,11 +831,13 @@ int dopt_bn_train_backward(int mode, const uint32_t* packed, const uint32_t* rel
     a.eps = eps;
     a.var_is_invstd = 0;
     a.dx = (uint16_t*)dx;
+    const int vw = bn_width(g, {{dy, bn_bytes(dy_dtype)}, {dx, 2}});
     (void)hipGetLastError();
-    dopt::launch_bn_bwd_reduce(a, dy_dtype, mode, group_size, bits, bn_width(g, {{dy, bn_bytes(dy_dtype)}}),
-                               (hipStream_t)stream, false);
-    dopt::launch_bn_bwd_dx(a, dy_dtype, mode, group_size, bits, bn_width(g, {{dy, bn_bytes(dy_dtype)}, {dx, 2}}),
-                           (hipStream_t)stream);
+    if (!dopt::launch_bn_bwd_whole(a, dy_dtype, mode, group_size, bits, vw, (hipStream_t)stream)) {
+        dopt::launch_bn_bwd_reduce(a, dy_dtype, mode, group_size, bits, bn_width(g, {{dy, bn_bytes(dy_dtype)}}),
+                                   (hipStream_t)stream, false);
+        dopt::launch_bn_bwd_dx(a, dy_dtype, mode, group_size, bits, vw, (hipStream_t)stream);
+    }
     return hip_status("bn_train_backward launch");
 }
 

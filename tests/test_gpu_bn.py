@@ -593,8 +593,6 @@ ROWS = [(32, 8, 7 * 7), (64, 5, 9), (32, 16, 10), (32, 3, 169), (96, 8, 11), (32
 def test_short_and_unaligned_rows(N, C, HW, dtype, kind, bits, shift):
     """The layer operators on [N, C, HW] equal, bit for bit, the same channels as one aligned row each ([1, C, N * HW]:
     8 elements per access), with x and dy at an element offset."""
-    if shift == 0 and HW % 4 == 0:
-        pytest.skip("aligned wide rows: covered above")
     gen = torch.Generator(device=DEV).manual_seed(N + HW + bits)
 
     def rows(t):  # [N, C, HW] -> [1, C, N * HW]
@@ -616,3 +614,40 @@ def test_short_and_unaligned_rows(N, C, HW, dtype, kind, bits, shift):
         if i in (0, 9):
             got = rows(got)
         assert torch.equal(got.view(torch.uint8), want.view(torch.uint8)), i
+
+
+# channels of one and two 8192-element chunks (the whole-channel kernels) at the edges of the chunks and of the lanes'
+# blocks, and one element group beyond them (the kernel pairs), in each access width
+CHANNELS = [(1, 3, 32), (1, 3, 8192), (1, 3, 8192 + 32), (1, 3, 16384), (1, 3, 16384 + 32), (2, 8, 4096 - 16), (8, 2, 4 * 257),
+            (96, 16, 49), (160, 8, 51), (224, 5, 49), (352, 3, 49)]
+
+
+@pytest.mark.parametrize("N,C,HW", CHANNELS)
+@pytest.mark.parametrize("dtype", DTYPES, ids=["bf16", "f32", "f16"])
+@pytest.mark.parametrize("kind,bits", [(1, 1), (1, 2), (1, 4), (2, 2), (3, 8)])
+def test_whole_channels_equal_the_operator_pairs(N, C, HW, dtype, kind, bits):
+    gen = torch.Generator(device=DEV).manual_seed(N + HW + bits)
+    x, dy = (torch.randn((N, C, HW), generator=gen, device=DEV).to(dtype) for _ in range(2))
+    w, b = torch.rand(C, generator=gen, device=DEV) + 0.5, torch.randn(C, generator=gen, device=DEV)
+    g, B = dict(M=N * HW, HW=HW, stride_n=C * HW, stride_c=HW), 64
+    s, q = ops.bn_fwd_reduce(x, **g, BLOCK_M=B, num_warps=8, num_stages=5)
+    if kind == 1:
+        y, packed, scale, xmin, mean, var = ops.bn_fwd_norm_quant_pack_fused(
+            x, s, q, w, b, None, None, **g, BLOCK_M=B, bits=bits, sync=False, avg_alam=False, alam_bits=0, num_warps=8,
+            num_stages=5)
+        mask = ()
+        dw, db = ops.bn_bwd_reduce_dequant_unpack_fused(packed, dy, scale, xmin, **g, BLOCK_M=B, bits=bits,
+                                                        avg_alam=False, alam_bits=0)
+        dx = ops.bn_bwd_dx_dequant_unpack_fused(packed, dy, scale, xmin, dw, db, w, var, **g, BLOCK_M=B, bits=bits,
+                                                sync=False, avg_alam=False, alam_bits=0)
+    else:
+        y, packed, mask, scale, xmin, mean, var = ops.bn_relu_fwd_norm_fused_quant_pack(
+            x, s, q, w, b, None, None, **g, relu=kind == 2, relu6=kind == 3, BLOCK_SIZE=B, BITS=bits, sync=False)
+        dw, db = ops.bn_relu_bwd_reduce_fused_dequant_unpack(packed, mask, dy, scale, xmin, **g, BLOCK_SIZE=B, BITS=bits)
+        dx = ops.bn_relu_bwd_dx_fused_dequant_unpack(packed, mask, dy, dw, db, w, var, scale, xmin, **g, BLOCK_SIZE=B,
+                                                     BITS=bits)
+    got = ops.bn_train_fwd(x, w, b, torch.zeros(0, device=DEV), torch.zeros(0, device=DEV), 0.1, B, bits, kind)
+    back = ops.bn_train_bwd(got[1], got[2] if kind != 1 else None, dy, got[3], got[4], w, got[6], B, bits, kind)
+    for i, (a, r) in enumerate(zip(got + back, (y, packed, mask, scale, xmin, mean, var, dx, dw, db))):
+        if not (i == 2 and kind == 1):
+            assert torch.equal(a.view(r.shape).view(torch.uint8), r.view(torch.uint8)), i
