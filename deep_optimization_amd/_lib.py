@@ -24,6 +24,7 @@ EXPORTS = (
     "dopt_abi_version",
     "dopt_last_error",
     "dopt_quant_pack",
+    "dopt_cast_quant_pack",
     "dopt_dequant_unpack",
     "dopt_pack_codes",
     "dopt_unpack_codes",
@@ -93,6 +94,8 @@ def lib() -> ctypes.CDLL:
         L.dopt_pack_codes.restype = i32
         L.dopt_unpack_codes.argtypes = [vp, i64, i32, i32, vp, vp]
         L.dopt_unpack_codes.restype = i32
+        L.dopt_cast_quant_pack.argtypes = [vp, i64, i32, i32, i32, f32, vp, vp, vp, vp, i32, vp]
+        L.dopt_cast_quant_pack.restype = i32
         L.dopt_fp8_gemm_nt.argtypes = [vp, vp, i64, i64, i64, i64, i64, f32, vp, i64, vp]
         L.dopt_fp8_gemm_nt.restype = i32
         L.dopt_fp8_gemm_kn.argtypes = [vp, vp, i64, i64, i64, i64, i64, i64, f32, vp, i64, vp]

@@ -14,7 +14,7 @@ import os
 import torch
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libdopt_torch.so")
-OPS = frozenset({"quant_pack", "quant_pack_tiles", "dequant_unpack", "dequant_unpack_tiles", "quant_pack_triton",
+OPS = frozenset({"quant_pack", "cast_quant_pack", "quant_pack_tiles", "dequant_unpack", "dequant_unpack_tiles", "quant_pack_triton",
                  "dequant_unpack_triton", "relu_fwd_fused_pack", "relu_bwd_fused_unpack", "bn_train_fwd",
                  "bn_train_bwd", "silu_fwd_quan_pack", "silu_bwd_fused_dequan_unpack", "gelu_bwd_fused_dequan_unpack",
                  "dw_gemm_any", "fp8_gemm_nt", "fp8_linear"})

@@ -195,6 +195,37 @@ quant_pack = _op(
         _meta3(x, x.shape[0], x.shape[1], bits, group_size, scale_dtype))
 
 
+def _cast_quant_pack(x, bits, group_size, clamp, clamp_alpha, squash, scale_dtype):
+    """fp32 x [N, G, group_size] -> (bf16 x, packed int32 [N*G, W], scale [N, G], min [N, G]): quant_pack of the bf16
+    rounding of x (nearest), which is returned too."""
+    _, nwords, _ = _bits_consts(bits, group_size)
+    if x.dim() != 3 or x.shape[-1] != group_size or x.dtype != torch.float32:
+        raise RuntimeError(f"cast_quant_pack expects a float32 x of shape [N, G, {group_size}], got {tuple(x.shape)} {x.dtype}")
+    if scale_dtype not in _META_CODE:
+        raise RuntimeError(f"cast_quant_pack: scale dtype must be float32 or bfloat16, got {scale_dtype}")
+    _require_cuda(x)
+    x = _aligned(x)
+    N, G, _ = x.shape
+    y = torch.empty(x.shape, dtype=torch.bfloat16, device=x.device)
+    packed = torch.empty((N * G, nwords), dtype=torch.int32, device=x.device)
+    scale = torch.empty((N, G), dtype=scale_dtype, device=x.device)
+    xmin = torch.empty((N, G), dtype=scale_dtype, device=x.device)
+    rc = _lib.lib().dopt_cast_quant_pack(x.data_ptr(), N * G, group_size, bits, _flags(clamp, squash), float(clamp_alpha),
+                                         y.data_ptr(), packed.data_ptr(), scale.data_ptr(), xmin.data_ptr(),
+                                         _META_CODE[scale_dtype], _stream(x))
+    _lib.check(rc, "cast_quant_pack")
+    return y, packed, scale, xmin
+
+
+cast_quant_pack = _op(
+    "cast_quant_pack(Tensor x, int bits, int group_size, bool clamp, float clamp_alpha, bool squash, "
+    "ScalarType scale_dtype) -> (Tensor, Tensor, Tensor, Tensor)",
+    _cast_quant_pack,
+    lambda x, bits, group_size, clamp, clamp_alpha, squash, scale_dtype:
+        (x.new_empty(x.shape, dtype=torch.bfloat16),
+         *_meta3(x, x.shape[0], x.shape[1], bits, group_size, scale_dtype)))
+
+
 def _tile_groups(shape, group_size: int):
     if len(shape) != 4:
         raise RuntimeError(f"tile layout expects a 4-D [N, C, H, W] tensor, got {tuple(shape)}")

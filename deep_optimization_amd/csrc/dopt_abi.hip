@@ -271,6 +271,37 @@ int dopt_quant_pack(const void* x, int x_dtype, int64_t n_groups, int group_size
     return hip_status("quant_pack launch");
 }
 
+int dopt_cast_quant_pack(const float* x, int64_t n_groups, int group_size, int bits, int flags, float clamp_alpha, void* y,
+                         uint32_t* packed, void* scale, void* minv, int meta_dtype, void* stream) {
+    int rc;
+    if ((rc = check_bits(bits))) return rc;
+    if ((rc = check_group(group_size))) return rc;
+    if (n_groups < 0 || n_groups >= (int64_t)1 << 31)
+        return fail(DOPT_EINVAL, "n_groups must be in [0, 2^31), got %lld", (long long)n_groups);
+    if (meta_dtype != DOPT_F32 && meta_dtype != DOPT_BF16)
+        return fail(DOPT_EINVAL, "scale/min dtype must be F32 or BF16, got code %d", meta_dtype);
+    if (flags & ~(DOPT_FLAG_CLAMP | DOPT_FLAG_SQUASH)) return fail(DOPT_EINVAL, "unknown flags 0x%x", flags);
+    if (n_groups == 0) return ok();
+    if (!x || !y || !packed || !scale || !minv) return fail(DOPT_EINVAL, "null pointer argument");
+    if (!aligned16(x) || !aligned16(y) || !aligned16(packed))
+        return fail(DOPT_EINVAL, "x, y and packed must be 16-byte aligned");
+    dopt::QuantPackArgs a{};
+    a.x = x;
+    a.y = y;
+    a.packed = packed;
+    a.scale = scale;
+    a.minv = minv;
+    a.n_groups = (uint32_t)n_groups;
+    a.clamp_alpha = clamp_alpha;
+    a.flags = (uint32_t)flags;
+    a.meta_bf16 = meta_dtype == DOPT_BF16;
+    (void)hipGetLastError();
+    if (dopt::launch_quant_pack_dt<dopt::DT_BF16>(a, bits, group_size, DOPT_ROUND_NEAREST, dopt::PRE_REF | dopt::PRE_CAST,
+                                                  (hipStream_t)stream))
+        return fail(DOPT_EUNSUPPORTED, "no casting quant-pack kernel for bits=%d g=%d", bits, group_size);
+    return hip_status("cast_quant_pack launch");
+}
+
 int dopt_dequant_unpack(const uint32_t* packed, const void* scale, const void* minv, int meta_dtype, int64_t n_groups,
                         int group_size, int bits, const int64_t* tile_nchw, void* y, int y_dtype, void* stream) {
     int rc;

@@ -57,11 +57,13 @@ namespace dopt {
 //   PRE_SQ16  PRE_REF's squash (with or without the clamp) of bf16 inputs at 1 and 2 bits, nearest
 //             rounding: the same words, scale and min bit for bit, from thresholds on the bf16 grid
 //             (squash16_pass below); a wave it cannot serve takes PRE_REF's per-element code
-enum { PRE_NONE = 0, PRE_REF = 1, PRE_GELU = 2, PRE_SILU = 3, PRE_SQ16 = 4 };
+//   PRE_CAST  (or'ed to PRE_REF or PRE_SQ16 of a bf16 kernel) the input is fp32: its bf16 rounding is
+//             written to y and quantized, so the cast's result is not read back for it
+enum { PRE_NONE = 0, PRE_REF = 1, PRE_GELU = 2, PRE_SILU = 3, PRE_SQ16 = 4, PRE_CAST = 8 };
 
 struct QuantPackArgs {
     const void* x;
-    void* y;  // activation output (PRE_GELU / PRE_SILU): bf16, same layout as x
+    void* y;  // activation output (PRE_GELU / PRE_SILU) or bf16(x) (PRE_CAST): bf16, same layout as x
     const float* noise;
     uint32_t* packed;
     void* scale;
@@ -318,9 +320,12 @@ __device__ __forceinline__ bool squash16_pass(const QuantPackArgs& a, const uint
     return true;
 }
 
-template <int DT, int BITS, int G, int RN, int UB, int LPG_, int P, int PRE, bool NT, bool TILED>
+template <int DT, int BITS, int G, int RN, int UB, int LPG_, int P, int PRE_, bool NT, bool TILED>
 __global__ __launch_bounds__(256) void quant_pack_kernel(QuantPackArgs a) {
     using C = QuantPackCfg<DT, BITS, G, RN, UB, LPG_, P>;
+    constexpr int PRE = PRE_ & ~PRE_CAST;
+    constexpr bool CAST = (PRE_ & PRE_CAST) != 0;
+    static_assert(!CAST || (DT == DT_BF16 && !TILED && RN == RN_NEAREST), "casting quantizer: flat, nearest, to bf16");
     constexpr int UE = C::UE, LOADS = C::LOADS, CPL = C::CPL, LPG = C::LPG, GPP = C::GPP, W = C::W;
     constexpr int UBITS = C::UBITS;
     constexpr int QMAX = (1 << BITS) - 1;
@@ -341,6 +346,8 @@ __global__ __launch_bounds__(256) void quant_pack_kernel(QuantPackArgs a) {
     // under a lane mask, merged with a default value, waits for its data before the next issues)
     uint4 raw[P][CPL][LOADS];
     uint4 nz[P][CPL][RN == RN_NOISE ? UE / 4 : 1];
+    uint4 wide[CAST ? P : 1][CAST ? CPL : 1][CAST ? 2 * LOADS : 1];  // the fp32 values of raw
+    (void)wide;
     #pragma unroll
     for (int p = 0; p < P; ++p) {
         const uint32_t r0 = g0 + p * GPP + slot;
@@ -349,11 +356,35 @@ __global__ __launch_bounds__(256) void quant_pack_kernel(QuantPackArgs a) {
         for (int i = 0; i < CPL; ++i) {
             const uint32_t e0 = (uint32_t)(i * LPG + li) * UE;
             #pragma unroll
-            for (int l = 0; l < LOADS; ++l)
-                raw[p][i][l] = ld16<NT>(xb + group_elem_index<G, TILED>(a, r, e0 + l * E16) * C::BYTES);
+            for (int l = 0; l < (CAST ? 2 : 1) * LOADS; ++l) {
+                if constexpr (CAST)
+                    wide[p][i][l] = ld16<NT>(xb + ((uint64_t)r * G + e0 + 4 * l) * 4);
+                else
+                    raw[p][i][l] = ld16<NT>(xb + group_elem_index<G, TILED>(a, r, e0 + l * E16) * C::BYTES);
+            }
             if constexpr (RN == RN_NOISE) {
                 #pragma unroll
                 for (int k = 0; k < UE / 4; ++k) nz[p][i][k] = ld16<NT>(a.noise + (uint64_t)r * G + e0 + 4 * k);
+            }
+        }
+    }
+
+    if constexpr (CAST) {
+        #pragma unroll
+        for (int p = 0; p < P; ++p) {
+            const uint32_t r = g0 + p * GPP + slot;
+            #pragma unroll
+            for (int i = 0; i < CPL; ++i) {
+                const uint32_t e0 = (uint32_t)(i * LPG + li) * UE;
+                #pragma unroll
+                for (int l = 0; l < LOADS; ++l) {
+                    const uint4 lo = wide[p][i][2 * l], hi = wide[p][i][2 * l + 1];
+                    raw[p][i][l] = make_uint4(pack_bf16x2(__uint_as_float(lo.x), __uint_as_float(lo.y)),
+                                              pack_bf16x2(__uint_as_float(lo.z), __uint_as_float(lo.w)),
+                                              pack_bf16x2(__uint_as_float(hi.x), __uint_as_float(hi.y)),
+                                              pack_bf16x2(__uint_as_float(hi.z), __uint_as_float(hi.w)));
+                    if (r < a.n_groups) st16<false>((char*)a.y + ((uint64_t)r * G + e0 + 8 * l) * 2, raw[p][i][l]);
+                }
             }
         }
     }

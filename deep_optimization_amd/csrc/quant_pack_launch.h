@@ -29,8 +29,10 @@ struct QuantPackShape {
     // the fastest kernels at 1-8 bits (four units, 108 VGPRs for GELU, ran 4-10% slower). The squashed
     // bf16 quantizer finds its thresholds once per lane, about 130 instructions, so a lane takes eight
     // units (never fewer than four lanes per group): bf16 [128,197,3072], g = 512, 2-bit, 42.0 / 29.9 /
-    // 27.6 us with two / four / eight units (51.3 us in the per-element form)
-    static constexpr int L0 = RN == RN_NOISE || RN == RN_PHILOX ? CPG : PRE == PRE_SQ16 ? (CPG < 32 ? 4 : CPG / 8) : CPG / 2;
+    // 27.6 us with two / four / eight units (51.3 us in the per-element form). The casting form moves three times
+    // the bytes per element and takes four, whose accesses lie closer together: fp32 [128,197,768], g = 256,
+    // 2-bit, 27.4 us with eight, 23.1 with four (the cast and the quantizer apart: 20.7 + 12.6)
+    static constexpr int L0 = RN == RN_NOISE || RN == RN_PHILOX ? CPG : PRE == PRE_SQ16 ? (CPG < 32 ? 4 : CPG / 8) : PRE == (PRE_SQ16 | PRE_CAST) ? (CPG < 16 ? 4 : CPG / 4) : CPG / 2;
     static constexpr int L1 = L0 < LPD ? LPD : L0;
     static constexpr int L2 = L1 < 2 ? 2 : L1;
     static constexpr int LPG = L2 > 64 ? 64 : L2;
@@ -49,7 +51,7 @@ static int qp_launch(const QuantPackArgs& a, hipStream_t s) {
                            linear_grid(blocks, 64 * C::WAVES), dim3(64 * C::WAVES), 0, s, a);
         return 0;
     }
-    if constexpr (G == 64 || G == 256 || G == 1024) {  // the square group sizes
+    if constexpr ((G == 64 || G == 256 || G == 1024) && !(PRE & PRE_CAST)) {  // the square group sizes
         hipLaunchKernelGGL((quant_pack_kernel<DT, BITS, G, RN, S::UB, S::LPG, S::P, PRE, false, true>),
                            linear_grid(blocks, 64 * C::WAVES), dim3(64 * C::WAVES), 0, s, a);
         return 0;
@@ -59,6 +61,17 @@ static int qp_launch(const QuantPackArgs& a, hipStream_t s) {
 
 template <int DT, int BITS, int G>
 static int qp_rn(const QuantPackArgs& a, int rn, int pre, hipStream_t s) {
+    if (pre == (PRE_REF | PRE_CAST)) {  // an fp32 input quantized as its bf16 rounding
+        if constexpr (DT == DT_BF16) {
+            if (rn != RN_NEAREST || a.tiled) return -1;
+            if constexpr (BITS <= 2) {
+                if ((a.flags & FL_SQUASH) && (!(a.flags & FL_CLAMP) || a.clamp_alpha >= 0.0f))
+                    return qp_launch<DT, BITS, G, RN_NEAREST, PRE_SQ16 | PRE_CAST>(a, s);
+            }
+            return qp_launch<DT, BITS, G, RN_NEAREST, PRE_REF | PRE_CAST>(a, s);
+        }
+        return -1;
+    }
     if (pre == PRE_REF) {  // the reference quantizer's clamp / squash, with any rounding
         switch (rn) {
             case RN_NEAREST:

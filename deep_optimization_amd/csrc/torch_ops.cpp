@@ -12,7 +12,7 @@
 // everything else RuntimeError. A device guard makes the tensors' device current for the call (the operators
 // whose Python implementation refuses tensors of another device refuse them here too).
 //
-// Operators: quant_pack, quant_pack_tiles, dequant_unpack, dequant_unpack_tiles,
+// Operators: quant_pack, cast_quant_pack, quant_pack_tiles, dequant_unpack, dequant_unpack_tiles,
 // quant_pack_triton, dequant_unpack_triton (AC/act_triton_kernel.py:336-395),
 // relu_fwd_fused_pack, relu_bwd_fused_unpack (AC/modules/activations/kernel_registration.py:42-94),
 // bn_train_fwd, bn_train_bwd (the compressed BatchNorm layers' one-call forward and backward),
@@ -134,6 +134,29 @@ std::tuple<Tensor, Tensor, Tensor> quant_pack(const Tensor& x, int64_t bits, int
     auto [p, s, m] = quant_pack_launch(x, N * G, bits, group_size, nullptr, clamp, clamp_alpha, squash, rounding,
                                        noise, seed, offset, scale_dtype);
     return {p, s.view({N, G}), m.view({N, G})};
+}
+
+std::tuple<Tensor, Tensor, Tensor, Tensor> cast_quant_pack(const Tensor& x_in, int64_t bits, int64_t group_size, bool clamp,
+                                                           double clamp_alpha, bool squash, ScalarType scale_dtype) {
+    const int64_t nwords = words_per_group(bits, group_size);
+    TORCH_CHECK(x_in.dim() == 3 && x_in.size(2) == group_size && x_in.scalar_type() == ScalarType::Float,
+                "cast_quant_pack expects a float32 x of shape [N, G, ", group_size, "], got ", x_in.sizes(), " ",
+                x_in.scalar_type());
+    TORCH_CHECK(scale_dtype == ScalarType::Float || scale_dtype == ScalarType::BFloat16,
+                "cast_quant_pack: scale dtype must be float32 or bfloat16, got ", scale_dtype);
+    require_cuda(x_in);
+    const c10::DeviceGuard guard(x_in.device());
+    const Tensor x = aligned(x_in);
+    const int64_t N = x.size(0), G = x.size(1);
+    const auto opts = x.options();
+    Tensor y = at::empty(x.sizes(), opts.dtype(at::kBFloat16));
+    Tensor packed = at::empty({N * G, nwords}, opts.dtype(at::kInt));
+    Tensor scale = at::empty({N, G}, opts.dtype(scale_dtype)), xmin = at::empty({N, G}, opts.dtype(scale_dtype));
+    check(dopt_cast_quant_pack(x.data_ptr<float>(), N * G, (int)group_size, (int)bits, flags(clamp, squash),
+                               (float)clamp_alpha, y.data_ptr(), (uint32_t*)packed.data_ptr(), scale.data_ptr(),
+                               xmin.data_ptr(), meta_code(scale_dtype), stream_of(x)),
+          "cast_quant_pack");
+    return {y, packed, scale, xmin};
 }
 
 // [N, C, H, W] in s x s spatial tiles: (N, G = C (H/s) (W/s))
@@ -659,6 +682,7 @@ std::tuple<Tensor, Tensor, Tensor> bn_train_bwd(const Tensor& packed_in, const s
 
 TORCH_LIBRARY_IMPL(act_lib, CUDA, m) {
     m.impl("quant_pack", &quant_pack);
+    m.impl("cast_quant_pack", &cast_quant_pack);
     m.impl("quant_pack_tiles", &quant_pack_tiles);
     m.impl("dequant_unpack", &dequant_unpack);
     m.impl("dequant_unpack_tiles", &dequant_unpack_tiles);

@@ -89,6 +89,27 @@ def unified_quantize(input, input_l, target_name, meta, clamp, clamp_alpha):
     return q_tensor, q_meta, input_l
 
 
+def cast_and_quantize(input, input_l, target_name, meta, clamp, clamp_alpha):
+    """unified_quantize of ``input.to(torch.bfloat16)`` and that tensor: (bf16 input, then unified_quantize's
+    results). A contiguous fp32 input in plain groups (no padding, tiles, runs of codes, or stochastic rounding) is
+    cast and quantized by one kernel, which reads it once; anything else casts first."""
+    m = meta[f"{target_name}"]
+    group_size = m["group_size"]
+    if (input.dtype == torch.float32 and input.is_cuda and input.is_contiguous() and not m["pack_only"]
+            and not m["act_padding"] and not m["AVG_ALAM"] and m.get("rounding", "nearest") in ("nearest", 0)
+            and not tile_layout_applies(input, group_size, False)):
+        groups, N, G, new_H, new_W, ori_shape, pad_elig, reshape_elig, channel_mean = spatical_aware_act_tensor_reshape(
+            input, Group_Size=group_size, act_padding=False, pack_only=False)
+        x16, out, scaler, xmin = torch.ops.act_lib.cast_quant_pack(
+            groups, m["bits"], group_size, clamp, clamp_alpha, m.get("squash", True),
+            m.get("scale_dtype", torch.bfloat16))
+        return (x16.view(input.shape), (out, scaler, xmin),
+                (m["bits"], m["pack_only"], group_size, m["act_padding"], N, G, new_H, new_W, pad_elig, reshape_elig,
+                 channel_mean, m["AVG_ALAM"], m["ALAM_BITS"], ori_shape), input_l)
+    input = input.to(torch.bfloat16)
+    return (input, *unified_quantize(input, input_l, target_name, meta, clamp, clamp_alpha))
+
+
 def dequantize(quantized_tensor, quantized_meta):
     """Reference module_utils.py:65-83: bf16 activations in the original shape."""
     q_input, q_scale, q_min = quantized_tensor
@@ -122,4 +143,4 @@ def unified_dequantize(ori_quantized_tensor, ori_quantized_meta, input_l):
     return x + F.interpolate(input_l, size=size, scale_factor=None, mode="nearest").to(torch.bfloat16)
 
 
-__all__ = ["quantize", "unified_quantize", "dequantize", "unified_dequantize", "default_act_tensor_reshape"]
+__all__ = ["quantize", "unified_quantize", "cast_and_quantize", "dequantize", "unified_dequantize", "default_act_tensor_reshape"]

@@ -36,7 +36,7 @@ from torch.autograd import Function
 from torch.nn.modules.utils import _pair, _single, _triple
 
 from ..dw_lib import dw_any_preferred, dw_gemm_supported
-from .module_utils import unified_dequantize, unified_quantize
+from .module_utils import cast_and_quantize, unified_dequantize, unified_quantize
 
 
 def _compute_dtype():
@@ -130,18 +130,24 @@ class _DOLinear(Function):
     def forward(ctx, input, weight, clamp_alpha, target_name, meta, ema_grad_meta, bias=None):
         dt = _compute_dtype()
         if dt is not None:
-            input = input.to(dt)
             weight_compute = weight.to(dt)
             bias_compute = None if bias is None else bias.to(dt)
         else:
             weight_compute, bias_compute = weight, bias
         m = meta[f"{target_name}"]
         input_l = None
-        if m.get("DIVISION") is not None and input.ndim not in (1, 2) and not m["pack_only"]:
-            k = min(input.shape[2], m["DIVISION"]["pool_kernel_size"])
-            input_l = F.avg_pool1d(input.to(torch.bfloat16), k, stride=k, padding=0)
-        q_tensor, q_meta, input_l = unified_quantize(input, input_l, target_name, meta, clamp=True,
-                                                     clamp_alpha=clamp_alpha)
+        division = m.get("DIVISION") is not None and input.ndim not in (1, 2) and not m["pack_only"]
+        if dt == torch.bfloat16 and not division:
+            input, q_tensor, q_meta, input_l = cast_and_quantize(input, None, target_name, meta, clamp=True,
+                                                                 clamp_alpha=clamp_alpha)
+        else:
+            if dt is not None:
+                input = input.to(dt)
+            if division:
+                k = min(input.shape[2], m["DIVISION"]["pool_kernel_size"])
+                input_l = F.avg_pool1d(input.to(torch.bfloat16), k, stride=k, padding=0)
+            q_tensor, q_meta, input_l = unified_quantize(input, input_l, target_name, meta, clamp=True,
+                                                         clamp_alpha=clamp_alpha)
         ctx.q_inputs_meta = q_meta
         ctx.meta = input.shape, ema_grad_meta, clamp_alpha, bias is not None
         # the packed codes can feed the weight-gradient GEMM directly when they are the flat

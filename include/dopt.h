@@ -90,6 +90,13 @@ int dopt_quant_pack(const void* x, int x_dtype, int64_t n_groups, int group_size
                     void* minv, int meta_dtype, void* stream);
 
 /*
+ * dopt_quant_pack of bf16(x) for an fp32 x [n_groups, group_size], nearest rounding, flat groups; bf16(x) is
+ * written to y (16-byte aligned). Codes, scale and min are those of a cast followed by dopt_quant_pack.
+ */
+int dopt_cast_quant_pack(const float* x, int64_t n_groups, int group_size, int bits, int flags, float clamp_alpha,
+                         void* y, uint32_t* packed, void* scale, void* minv, int meta_dtype, void* stream);
+
+/*
  * Unpack + dequantize: y = fma(float(q), scale, min), rounded once to y_dtype (F32 or BF16).
  * Replaces act_lib::dequant_unpack_triton (act_triton_kernel.py:372-395, kernel :174-241) and
  * the cpp_extension unpack1..unpack8 entry points (cpp_extension/bind.cpp:54-58,

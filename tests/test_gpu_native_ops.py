@@ -214,3 +214,61 @@ def test_refused_operands():
         for f in (native, python):
             with pytest.raises(RuntimeError):
                 f(*args)
+
+
+@pytest.mark.parametrize("bits", [1, 2, 4, 8])
+@pytest.mark.parametrize("g", [64, 128, 256, 512, 1024])
+@pytest.mark.parametrize("N,G", [(1, 1), (3, 7), (5, 67)])
+def test_cast_quant_pack(bits, g, N, G):
+    """One call equals the cast followed by quant_pack, bit for bit, and the Python implementation: values over the
+    whole exponent range, constant groups, infinities, NaN and signed zeros among them."""
+    x = rnd((N, G, g), bits + g, dtype=torch.float32)
+    x[0, 0, ::3] *= 1e-30
+    x[-1, -1] = 1.5
+    if N > 1:
+        x[1, 0, 5], x[1, 1, 7], x[1, 2, 9] = float("inf"), float("-inf"), float("nan")
+        x[1, 3, ::2], x[1, 4] = -0.0, 3.4e38
+        x[2, 0] = torch.exp2(torch.linspace(-140.0, 120.0, g, device=DEV))
+    for clamp, squash, sdt in ((True, True, torch.bfloat16), (False, True, torch.float32), (True, False, torch.bfloat16),
+                               (False, False, torch.float32)):
+        got = ops.cast_quant_pack(x, bits, g, clamp, 2.5, squash, sdt)
+        same(got, act_lib._cast_quant_pack(x, bits, g, clamp, 2.5, squash, sdt))
+        x16 = x.to(torch.bfloat16)
+        nan = x16.isnan()
+        assert torch.equal(nan, got[0].isnan())
+        same(got[0].masked_fill(nan, 0.0), x16.masked_fill(nan, 0.0))
+        want = ops.quant_pack(x16, bits, g, clamp, 2.5, squash, 0, None, 0, 0, sdt)
+        for i, (a, b) in enumerate(zip(got[1:], want)):
+            if i == 0:
+                same(a, b)
+            else:  # a group of NaN: whatever its NaN's bits
+                assert torch.equal(a.isnan(), b.isnan())
+                same(torch.nan_to_num(a, 0.0), torch.nan_to_num(b, 0.0))
+
+
+@pytest.mark.parametrize("shape,bits", [((4, 50, 384), 2), ((5, 768), 1), ((3, 7, 128), 8), ((3, 7, 100), 2)])
+def test_linear_layer_fp32_input(shape, bits):
+    """The compressed Linear layer on an fp32 input under autocast (one kernel casts and quantizes; a padded one casts
+    first) saves and returns what it does on the input cast beforehand; a transposed input too."""
+    from deep_optimization_amd.controller import layer_group_meta
+    from deep_optimization_amd.modules.ops import _DOLinear
+
+    meta = {"l": {"bits": bits, "pack_only": False, "AVG_ALAM": False, "ALAM_BITS": 0, "DIVISION": None,
+                  **layer_group_meta(shape, bits)}}
+    w = rnd((256, shape[-1]), 5, torch.float32)
+    bias = rnd((256,), 6, torch.float32)
+    base = rnd(shape, 7, torch.float32)
+    if len(shape) == 3:
+        views = (base, base.transpose(0, 1).contiguous().transpose(0, 1))
+    else:
+        views = (base, base.t().contiguous().t())
+    for view in views:
+        out = []
+        for x in (view.to(torch.bfloat16), view):  # (the cast keeps the strides, and with them the product's kernel)
+            x = x.detach().requires_grad_(True)
+            wi, bi = w.clone().requires_grad_(True), bias.clone().requires_grad_(True)
+            with torch.autocast("cuda", dtype=torch.bfloat16):
+                y = _DOLinear.apply(x, wi, 3.0, "l", meta, None, bi)
+            y.backward(rnd(y.shape, 8))
+            out.append(tuple(t.detach().contiguous() for t in (y, x.grad.float(), wi.grad, bi.grad)))
+        same(out[1], out[0])
