@@ -292,7 +292,7 @@ def test_errors():
 # ----------------------------------------------------------------------------- avg_alam
 # (shape, BLOCK_M, bits, alam_bits): run lengths dividing the group's code words (1: the plain
 # codes, noise in the reduce only; 16 and 64: runs spanning 2 and 8 lanes), every access width
-# (8 at 16x16 / 28x28, 4 at 14x14, 2 at 5x10, 1 at 7x7), groups of 32..256, and channels whose last
+# (8 at 16x16 / 28x28, 4 at 14x14, 8 at any element at 5x10 and 7x7), groups of 32..256, and channels whose last
 # wave of 512 elements lies partly past M (7x7: M = 1568); each in bf16, fp32 and fp16
 ACASES = [((4, 16, 16, 16), 64, 2, 2), ((4, 16, 16, 16), 64, 8, 8), ((16, 8, 14, 14), 128, 1, 2),
           ((16, 32, 14, 14), 128, 4, 4), ((32, 16, 28, 28), 512, 2, 16), ((32, 16, 28, 28), 512, 8, 64),
