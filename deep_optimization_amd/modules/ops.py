@@ -172,7 +172,7 @@ class _DOLinear(Function):
         C_in, C_out = input_shape[-1], dy.shape[-1]
         dy_flat = dy.reshape(-1, C_out)
         out_dtype = ctx.w_dtype if ctx.w_dtype in (torch.float32, torch.bfloat16) else torch.float32
-        kernel = dy.dtype == torch.bfloat16
+        kernel = dy.dtype == torch.bfloat16 and not ctx.q_inputs_meta[1]  # (pack-only codes are restored as int8)
         from_codes = ctx.fused_unpack and q1.dtype == torch.bfloat16 and dw_gemm_supported(C_out, C_in)
         if kernel and from_codes:
             # weight (and bias) gradient on the gfx950 split-K GEMM for K-outer operands, in the

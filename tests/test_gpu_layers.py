@@ -77,6 +77,25 @@ def test_do_linear(bits, shape, autocast, cout, fused):
     assert rel_err(layer.bias.grad, dyf.sum(0)) <= 1e-2
 
 
+@pytest.mark.parametrize("bias", [True, False])
+@pytest.mark.parametrize("cin,cout", [(384, 200), (512, 256), (320, 100)])
+def test_do_linear_pack_only(cin, cout, bias):
+    """A pack-only layer saves its input's codes alone and restores them as int8: the weight gradient is
+    dy^T . codes for widths of every route (multiples of 8 and of 256, and neither)."""
+    torch.manual_seed(cin + cout)
+    shape = (4, 320, cin)
+    layer = DOLinear(cin, cout, target_name="fc", meta=meta_for("fc", shape, 2, pack_only=True), bias=bias, device=DEV).train()
+    x = torch.randint(0, 2, shape, device=DEV).float().requires_grad_(True)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        y = layer(x)
+    dy = torch.randn_like(y)
+    y.backward(dy)
+    dyf = dy.float().reshape(-1, cout)
+    assert rel_err(layer.weight.grad, dyf.t() @ x.detach().reshape(-1, cin)) <= 1e-2
+    if bias:
+        assert rel_err(layer.bias.grad, dyf.sum(0)) <= 1e-2
+
+
 @pytest.mark.parametrize("rounding", ["stochastic", "stochastic_noise"])
 def test_do_linear_stochastic_rounding_meta(rounding):
     """The per-layer meta keys 'rounding' = 'stochastic' (Philox) / 'stochastic_noise' reach the
