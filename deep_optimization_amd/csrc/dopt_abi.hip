@@ -436,8 +436,13 @@ int dopt_fp8_gemm_nt(const uint8_t* A, const uint8_t* B, int64_t M, int64_t N, i
     return hip_status("fp8_gemm launch");
 }
 
+// The largest row-major B rows and tile counts that dopt_fp8_gemm_kn takes (32-bit offsets, one launch)
+static bool fp8_kn_ldb(int64_t ldb) { return ldb < (1 << 23); }
+static bool fp8_kn_tiles(int64_t M, int64_t N) { return (M + 31) / 32 * ((N + 63) / 64) < ((int64_t)1 << 31); }
+
 int dopt_fp8_gemm_kn_preferred(int64_t M, int64_t N, int64_t K) {
-    return M > 0 && N > 0 && K > 0 && dopt::fp8_gemm_kn_preferred(M, N, K);
+    return M > 0 && N > 0 && K > 0 && fp8_kn_ldb((N + 15) / 16 * 16) && fp8_kn_tiles(M, N) &&
+           dopt::fp8_gemm_kn_preferred(M, N, K);
 }
 
 int dopt_fp8_gemm_kn(const uint8_t* A, const uint8_t* B, int64_t M, int64_t N, int64_t K, int64_t b_rows, int64_t lda,
@@ -455,10 +460,10 @@ int dopt_fp8_gemm_kn(const uint8_t* A, const uint8_t* B, int64_t M, int64_t N, i
                     "fp8_gemm_kn needs 16-byte aligned A and B, multiples of 16 lda >= K and ldb >= N, a 2-byte aligned C "
                     "and ldc >= N (got lda=%lld ldb=%lld ldc=%lld K=%lld N=%lld)",
                     (long long)lda, (long long)ldb, (long long)ldc, (long long)K, (long long)N);
-    if (lda >= (1 << 23) || ldb >= (1 << 23))
+    if (lda >= (1 << 23) || !fp8_kn_ldb(ldb))
         return fail(DOPT_EINVAL, "fp8 GEMM row strides must be below 2^23 bytes (32-bit tile offsets), got %lld, %lld",
                     (long long)lda, (long long)ldb);
-    if ((M + 31) / 32 * ((N + 63) / 64) >= ((int64_t)1 << 31))
+    if (!fp8_kn_tiles(M, N))
         return fail(DOPT_EINVAL, "fp8 GEMM output too large: %lld x %lld", (long long)M, (long long)N);
     (void)hipGetLastError();
     dopt::launch_fp8_gemm_kn(A, B, M, N, K, b_rows, lda, ldb, out_scale, (uint16_t*)C, ldc, (hipStream_t)stream);

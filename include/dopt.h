@@ -166,7 +166,8 @@ int dopt_fp8_gemm_nt(const uint8_t* A, const uint8_t* B, int64_t M, int64_t N, i
  * each readable up to N rounded up to a multiple of 16 (what lies past N is not used).
  * lda >= K and ldb >= N multiples of 16 and < 2^23, A and B 16-byte aligned, C as above.
  * dopt_fp8_gemm_kn_preferred: 1 where this is estimated to be faster than packing B for
- * dopt_fp8_gemm_nt first (outputs below the sizes that the 256 x 256 tiles need).
+ * dopt_fp8_gemm_nt first (outputs below the sizes that the 256 x 256 tiles need); 0 for every N whose rows
+ * dopt_fp8_gemm_kn does not take.
  */
 int dopt_fp8_gemm_kn(const uint8_t* A, const uint8_t* B, int64_t M, int64_t N, int64_t K, int64_t b_rows,
                      int64_t lda, int64_t ldb, float out_scale, void* C, int64_t ldc, void* stream);

@@ -87,6 +87,14 @@ def test_row_major_b(M, N, K, padded):
         assert torch.equal(got, c[:M, :N])
 
 
+@pytest.mark.parametrize("M,N,K", [(1, (1 << 23) + 5, 16), (2, 1 << 23, 16), (1, (1 << 23) - 16, 16)])
+def test_row_major_b_longest_rows(M, N, K):
+    """Rows of B around 2^23 bytes: past what the kernels read as it lies, fp8_linear packs it."""
+    gen = torch.Generator(device=DEV).manual_seed(N)
+    a, b = fp8((M, K), gen), fp8((K, N), gen)
+    check(torch.ops.act_lib.fp8_linear(a, b, 0.125), a, b.t(), 0.125)
+
+
 def test_row_major_b_refuses():
     a, b = (torch.zeros(4096, dtype=torch.uint8, device=DEV) for _ in range(2))
     c = torch.zeros((16, 32), dtype=torch.bfloat16, device=DEV)

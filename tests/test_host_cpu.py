@@ -55,6 +55,12 @@ class TestValidationWithoutDevice:
                                           a["noise"], a["seed"], a["off"], a["flags"], a["alpha"], a["packed"],
                                           a["scale"], a["minv"], a["meta"], a["stream"])
 
+    @pytest.mark.parametrize("N", [(1 << 23) - 15, 1 << 23, (1 << 23) + 1, 1 << 25])
+    def test_row_major_b_is_not_preferred_past_its_row_limit(self, N):
+        for M in (1, 8, 64, 512):
+            for K in (16, 256, 4096):
+                assert _lib.lib().dopt_fp8_gemm_kn_preferred(M, N, K) == 0, (M, N, K)
+
     def test_bad_bits_is_value_error(self):
         assert self.qp(bits=3) == _lib.EBITS
         with pytest.raises(ValueError, match="bits must be one of"):
