@@ -31,6 +31,7 @@ EXPORTS = (
     "dopt_fp8_gemm_nt",
     "dopt_fp8_gemm_kn",
     "dopt_fp8_gemm_kn_preferred",
+    "dopt_fp8_gemm_kn_copy_preferred",
     "dopt_fp8_pack_kmajor",
     "dopt_fp8_pack_kmajor_padded",
     "dopt_relu_pack",
@@ -102,6 +103,8 @@ def lib() -> ctypes.CDLL:
         L.dopt_fp8_gemm_kn.restype = i32
         L.dopt_fp8_gemm_kn_preferred.argtypes = [i64, i64, i64]
         L.dopt_fp8_gemm_kn_preferred.restype = i32
+        L.dopt_fp8_gemm_kn_copy_preferred.argtypes = [i64, i64, i64]
+        L.dopt_fp8_gemm_kn_copy_preferred.restype = i32
         L.dopt_fp8_pack_kmajor.argtypes = [vp, i64, i64, i64, i64, vp, i64, vp]
         L.dopt_fp8_pack_kmajor.restype = i32
         L.dopt_fp8_pack_kmajor_padded.argtypes = [vp, i64, i64, i64, i64, vp, i64, i64, vp]

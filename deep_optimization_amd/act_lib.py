@@ -496,9 +496,11 @@ def _fp8_linear(a, b, out_scale):
         return c.zero_()
     k_pad = (K + 15) // 16 * 16
     ta, lda = _kmajor(a.view(torch.uint8), M, K, a.stride(0), a.stride(1), k_pad)
-    if b.stride(1) == 1 and _lib.lib().dopt_fp8_gemm_kn_preferred(M, N, k_pad):
-        tb, ldb = b.view(torch.uint8), b.stride(0)
-        if ldb % 16 or not N <= ldb < (1 << 23) or N % 16 or b.data_ptr() % 16:  # a copy with aligned rows
+    tb, ldb = b.view(torch.uint8), b.stride(0)
+    copied = ldb % 16 or not N <= ldb < (1 << 23) or N % 16 or b.data_ptr() % 16
+    L = _lib.lib()
+    if b.stride(1) == 1 and (L.dopt_fp8_gemm_kn_copy_preferred if copied else L.dopt_fp8_gemm_kn_preferred)(M, N, k_pad):
+        if copied:  # into aligned rows
             ldb = (N + 15) // 16 * 16
             tb = torch.empty((K, ldb), dtype=torch.uint8, device=a.device)
             rc = _lib.lib().dopt_fp8_pack_kmajor_padded(b.data_ptr(), K, N, b.stride(0), 1, tb.data_ptr(), ldb, ldb,

@@ -19,7 +19,7 @@ int launch_fp8_gemm_nt(const uint8_t* A, const uint8_t* B, int64_t M, int64_t N,
                        int64_t ldb, float out_scale, uint16_t* C, int64_t ldc, hipStream_t s);
 int launch_fp8_gemm_kn(const uint8_t* A, const uint8_t* B, int64_t M, int64_t N, int64_t K, int64_t b_rows, int64_t lda,
                        int64_t ldb, float out_scale, uint16_t* C, int64_t ldc, hipStream_t s);
-bool fp8_gemm_kn_preferred(int64_t M, int64_t N, int64_t K);
+bool fp8_gemm_kn_preferred(int64_t M, int64_t N, int64_t K, bool copied);
 int launch_fp8_pack(const uint8_t* src, int64_t rows, int64_t cols, int64_t stride_r, int64_t stride_c, uint8_t* dst,
                     int64_t ld_dst, int64_t cols_out, hipStream_t s);
 int launch_relu_pack(const void* x, int dt, void* y, uint32_t* packed, uint64_t n, int bits, bool relu6, hipStream_t s);
@@ -440,10 +440,14 @@ int dopt_fp8_gemm_nt(const uint8_t* A, const uint8_t* B, int64_t M, int64_t N, i
 static bool fp8_kn_ldb(int64_t ldb) { return ldb < (1 << 23); }
 static bool fp8_kn_tiles(int64_t M, int64_t N) { return (M + 31) / 32 * ((N + 63) / 64) < ((int64_t)1 << 31); }
 
-int dopt_fp8_gemm_kn_preferred(int64_t M, int64_t N, int64_t K) {
+static int fp8_kn_preferred(int64_t M, int64_t N, int64_t K, bool copied) {
     return M > 0 && N > 0 && K > 0 && fp8_kn_ldb((N + 15) / 16 * 16) && fp8_kn_tiles(M, N) &&
-           dopt::fp8_gemm_kn_preferred(M, N, K);
+           dopt::fp8_gemm_kn_preferred(M, N, K, copied);
 }
+
+int dopt_fp8_gemm_kn_preferred(int64_t M, int64_t N, int64_t K) { return fp8_kn_preferred(M, N, K, false); }
+
+int dopt_fp8_gemm_kn_copy_preferred(int64_t M, int64_t N, int64_t K) { return fp8_kn_preferred(M, N, K, true); }
 
 int dopt_fp8_gemm_kn(const uint8_t* A, const uint8_t* B, int64_t M, int64_t N, int64_t K, int64_t b_rows, int64_t lda,
                      int64_t ldb, float out_scale, void* C, int64_t ldc, void* stream) {

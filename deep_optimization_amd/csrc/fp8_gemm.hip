@@ -120,12 +120,17 @@ int launch_fp8_gemm_kn(const uint8_t* A, const uint8_t* B, int64_t M, int64_t N,
 // as it lies: 985 x 768 x 1536 8.5 -> 5.5, 64 x 4096 x 4096 17.1 -> 6.7, 1024^3 7.8 -> 4.8, 2048^3
 // 18.0 -> 11.4, 8192 x 1024 x 1024 17.6 -> 15.3; the other way at 3000^3 (50.7 against 55.8) and 4096^3
 // (57.4 against 72.2), where the 256 x 256 tiles win.
-bool fp8_gemm_kn_preferred(int64_t M, int64_t N, int64_t K) {
+// A B that would have to be copied into aligned rows first (`copied`) is passed over once either way, by the copy
+// about 0.3 us faster than by the transpose: the row-major kernel has to be that close to the other one. Over 230
+// random odd N from 17 to 8191 (captured calls, copy or transpose included) the faster way is lost by 1.0% in the
+// geometric mean and by more than 5% on 18; with the comparison above it was 4.8% and 60 (16 x 1001 x 8192 24.2
+// against 14.4 us packed, 64 x 4097 x 4096 19.2 against 17.4, 2500 x 2501 x 1000 24.9 against 21.7).
+bool fp8_gemm_kn_preferred(int64_t M, int64_t N, int64_t K, bool copied) {
     const int n_cu = device_cu_count();
     float kn, nt;
     plan(M, N, K, n_cu, true, &kn);
     plan(M, N, K, n_cu, false, &nt);
-    return kn < nt + 3.0f + (float)N * (float)K * (1.0f / 3.2e6f);
+    return kn < nt + (copied ? 0.3f : 3.0f + (float)N * (float)K * (1.0f / 3.2e6f));
 }
 
 }  // namespace dopt

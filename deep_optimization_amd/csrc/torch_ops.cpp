@@ -528,10 +528,11 @@ Tensor fp8_linear(const Tensor& a, const Tensor& b, double out_scale) {
     if (K == 0) return c.zero_();
     const int64_t k_pad = (K + 15) / 16 * 16;
     const auto [ta, lda] = kmajor(a, M, K, a.stride(0), a.stride(1), k_pad);
-    if (b.stride(1) == 1 && dopt_fp8_gemm_kn_preferred(M, N, k_pad)) {
+    int64_t ldb = b.stride(0);
+    const bool copied = ldb % 16 || ldb < N || ldb >= (1 << 23) || N % 16 || reinterpret_cast<uintptr_t>(b.data_ptr()) % 16;
+    if (b.stride(1) == 1 && (copied ? dopt_fp8_gemm_kn_copy_preferred : dopt_fp8_gemm_kn_preferred)(M, N, k_pad)) {
         Tensor tb = b;
-        int64_t ldb = b.stride(0);
-        if (ldb % 16 || ldb < N || ldb >= (1 << 23) || N % 16 || reinterpret_cast<uintptr_t>(b.data_ptr()) % 16) {
+        if (copied) {
             ldb = (N + 15) / 16 * 16;  // a copy with aligned rows
             tb = at::empty({K, ldb}, b.options().dtype(at::kByte));
             check(dopt_fp8_pack_kmajor_padded((const uint8_t*)b.data_ptr(), K, N, b.stride(0), 1, (uint8_t*)tb.data_ptr(),
@@ -543,8 +544,8 @@ Tensor fp8_linear(const Tensor& a, const Tensor& b, double out_scale) {
               "fp8_linear");
         return c;
     }
-    const auto [tb, ldb] = kmajor(b, N, K, b.stride(1), b.stride(0), k_pad);
-    check(dopt_fp8_gemm_nt((const uint8_t*)ta.data_ptr(), (const uint8_t*)tb.data_ptr(), M, N, k_pad, lda, ldb,
+    const auto [tb, ldk] = kmajor(b, N, K, b.stride(1), b.stride(0), k_pad);
+    check(dopt_fp8_gemm_nt((const uint8_t*)ta.data_ptr(), (const uint8_t*)tb.data_ptr(), M, N, k_pad, lda, ldk,
                            (float)out_scale, c.data_ptr(), N, stream_of(a)),
           "fp8_linear");
     return c;

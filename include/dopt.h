@@ -167,11 +167,13 @@ int dopt_fp8_gemm_nt(const uint8_t* A, const uint8_t* B, int64_t M, int64_t N, i
  * lda >= K and ldb >= N multiples of 16 and < 2^23, A and B 16-byte aligned, C as above.
  * dopt_fp8_gemm_kn_preferred: 1 where this is estimated to be faster than packing B for
  * dopt_fp8_gemm_nt first (outputs below the sizes that the 256 x 256 tiles need); 0 for every N whose rows
- * dopt_fp8_gemm_kn does not take.
+ * dopt_fp8_gemm_kn does not take. dopt_fp8_gemm_kn_copy_preferred: the same where B's rows are not aligned, so
+ * that it has to be copied (dopt_fp8_pack_kmajor_padded) before it can be read this way.
  */
 int dopt_fp8_gemm_kn(const uint8_t* A, const uint8_t* B, int64_t M, int64_t N, int64_t K, int64_t b_rows,
                      int64_t lda, int64_t ldb, float out_scale, void* C, int64_t ldc, void* stream);
 int dopt_fp8_gemm_kn_preferred(int64_t M, int64_t N, int64_t K);
+int dopt_fp8_gemm_kn_copy_preferred(int64_t M, int64_t N, int64_t K);
 
 /*
  * Layout conversion for dopt_fp8_gemm_nt: dst[r * ld_dst + c] = src[r * stride_r + c * stride_c]

@@ -95,6 +95,15 @@ def test_row_major_b_longest_rows(M, N, K):
     check(torch.ops.act_lib.fp8_linear(a, b, 0.125), a, b.t(), 0.125)
 
 
+@pytest.mark.parametrize("M,N,K", [(16, 1001, 520), (64, 100, 2000), (300, 513, 65)])
+def test_unaligned_row_major_b(M, N, K):
+    """fp8_linear of a B in unaligned rows, copied or packed: the product either way."""
+    gen = torch.Generator(device=DEV).manual_seed(N)
+    a, wide = fp8((M, K), gen), fp8((K, N + 7), gen)
+    for b in (wide[:, :N].contiguous(), wide[:, 3:N + 3], wide[:, :1].expand(K, N), wide[:1, :N].expand(K, N)):
+        check(torch.ops.act_lib.fp8_linear(a, b, 0.125), a, b.t(), 0.125)
+
+
 def test_row_major_b_refuses():
     a, b = (torch.zeros(4096, dtype=torch.uint8, device=DEV) for _ in range(2))
     c = torch.zeros((16, 32), dtype=torch.bfloat16, device=DEV)
