@@ -483,8 +483,8 @@ int dopt_fp8_pack_kmajor_padded(const uint8_t* src, int64_t rows, int64_t cols, 
                                 uint8_t* dst, int64_t ld_dst, int64_t cols_out, void* stream) {
     if (rows < 0 || cols < 0 || stride_r < 0 || stride_c < 0)
         return fail(DOPT_EINVAL, "fp8 pack: negative extent or stride");
-    if (rows == 0 || cols == 0) return ok();
-    if (!src || !dst) return fail(DOPT_EINVAL, "null pointer argument");
+    if (rows == 0 || (cols == 0 && cols_out <= 0)) return ok();
+    if ((cols > 0 && !src) || !dst) return fail(DOPT_EINVAL, "null pointer argument");
     if (ld_dst < cols) return fail(DOPT_EINVAL, "fp8 pack: ld_dst (%lld) < cols (%lld)", (long long)ld_dst, (long long)cols);
     if (cols_out < cols || cols_out > ld_dst || cols_out - cols > 15)
         return fail(DOPT_EINVAL, "fp8 pack: %lld columns out of %lld: at most 15 more, and within ld_dst (%lld)",

@@ -141,3 +141,15 @@ def test_pack_kmajor(rows, cols, layout, shift):
             _lib.check(rc, "fp8_pack_kmajor_padded")
             assert torch.equal(dst[:, :cols], view)
             assert bool((dst[:, cols:out] == 0).all()) and bool((dst[:, out:] == 0xAB).all())
+
+
+@pytest.mark.parametrize("strides", [(1, 40), (40, 1), (40, 2)], ids=["transposed", "rows", "gather"])
+def test_pack_kmajor_padded_without_columns(strides):
+    """No columns in, up to 15 zero columns out."""
+    src = torch.full((4096,), 7, dtype=torch.uint8, device=DEV)
+    for out in (1, 15):
+        dst = torch.full((33, 20), 0xAB, dtype=torch.uint8, device=DEV)
+        rc = _lib.lib().dopt_fp8_pack_kmajor_padded(src.data_ptr(), 33, 0, *strides, dst.data_ptr(), 20, out,
+                                                    torch.cuda.current_stream().cuda_stream)
+        _lib.check(rc, "fp8_pack_kmajor_padded")
+        assert bool((dst[:, :out] == 0).all()) and bool((dst[:, out:] == 0xAB).all())
