@@ -22,7 +22,8 @@ struct DwArgs {
     int64_t M, N, K;
     int64_t kt_per_split;     // set by the launcher
     int splits;               // splits with work (set by the launcher)
-    float* partial;           // workspace: [splits][M][N] fp32, then [splits][M] for db
+    float* partial;           // workspace: [splits][M][N] fp32, then [splits][M] for db; one split: the fp32 result
+    uint16_t* out16;          // the bf16 result, of the kernels that write it in place of partial
     float* db_partial;        // set by the launcher
 };
 

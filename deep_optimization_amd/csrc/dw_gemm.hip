@@ -357,12 +357,16 @@ struct V2Codes {
 // is no multiple of 32 had gone through dw_gemm_kernel (768 x 3072 over 3645 tokens 51 -> 40 us), and other M, N
 // through torch's product and sum (384 x 1536 over 6304 tokens 68 -> 25 us, 640 x 640 over 12000 100 -> 23 us).
 // BNT: output columns per workgroup tile (256, or 128 for RAG).
-template <int BITS, bool DB, int NW, int BMT, int BNT = 256, bool RAG = false>
+// O16 (bf16 x_hat, one split): the result goes out in bf16, not as an fp32 partial matrix that a second kernel
+// rounds, 10 bytes an element for 2 (4096 x 4096 over 333 tokens 41.8 -> 22.5 us, 10000 x 512 over 64 with db
+// 21.1 -> 10.3; torch's product and sum take 12.9 there).
+template <int BITS, bool DB, int NW, int BMT, int BNT = 256, bool RAG = false, bool O16 = false>
 __global__ __launch_bounds__(64 * NW, 1) void dw_gemm_v2_kernel(DwArgs a) {
     static_assert(BITS == 0 || BITS == 1 || BITS == 2 || BITS == 4, "bf16, or 1/2/4-bit codes");
     static_assert(NW == 4 || (NW == 8 && BITS == 0), "8 waves for bf16 x_hat only");
     static_assert(BNT == 256 || (BNT == 128 && RAG), "narrow x_hat tiles for the ragged kernel only");
     static_assert(!RAG || BITS == 0, "ragged shapes: bf16 x_hat only");
+    static_assert(!O16 || BITS == 0, "bf16 results: bf16 x_hat only");
     using CS = V2Codes<BITS>;
     constexpr int WN = NW / 2;            // waves along n
     constexpr int CW = BNT / WN;          // columns per wave
@@ -654,8 +658,27 @@ __global__ __launch_bounds__(64 * NW, 1) void dw_gemm_v2_kernel(DwArgs a) {
     // the trailing (unused) loads land before the kernel ends
     __builtin_amdgcn_s_waitcnt(0);
 
-    float* P = a.partial + (int64_t)split * a.M * a.N;
-    if constexpr (RAG) {
+    if constexpr (O16) {
+        // the one split's tile, rounded: rows past M lie past the end of the result, columns past N load the mask
+        const int64_t left = ((a.M - m0) * a.N - n0) * 2;
+        const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(
+            (void*)(a.out16 + m0 * a.N + n0), (short)0, (int)min(left, (int64_t)0x7FFFFF00), 0x00020000);
+        const uint32_t rowb = (uint32_t)a.N * 2u;
+#pragma unroll
+        for (int j = 0; j < TNW; ++j) {
+            const int64_t col = wn * CW + j * 32 + (lane & 31);
+            const uint32_t off = ((uint32_t)(wm * RW + 4 * (lane >> 5)) * rowb + (uint32_t)col * 2u) |
+                                 (n0 + col < a.N ? 0u : BUF_OOB);
+#pragma unroll
+            for (int i = 0; i < TMW; ++i)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    const uint32_t o = off + (uint32_t)(i * 32 + 8 * (v >> 2) + (v & 3)) * rowb;
+                    __builtin_amdgcn_raw_buffer_store_b16(to_bf16(acc[i][j][v]), rp, o, 0, 0);
+                }
+        }
+    } else if constexpr (RAG) {
+        float* P = a.partial + (int64_t)split * a.M * a.N;
         // rows past M lie past the end of the split's partial matrix, columns past N load the mask: neither
         // is stored (and no branch per element)
         const int64_t left = ((a.M - m0) * a.N - n0) * 4;
@@ -676,6 +699,7 @@ __global__ __launch_bounds__(64 * NW, 1) void dw_gemm_v2_kernel(DwArgs a) {
                 }
         }
     } else {
+        float* P = a.partial + (int64_t)split * a.M * a.N;
 #pragma unroll
         for (int i = 0; i < TMW; ++i)
 #pragma unroll
@@ -818,9 +842,6 @@ int64_t dw_workspace_floats(int64_t M, int64_t N, int64_t K) {
 
 int launch_dw_gemm(DwArgs a, int mode, bool with_db, float* out32, uint16_t* out16, float* db, hipStream_t st) {
     const int splits = dw_splits(a.M, a.N, a.K);
-    // one split and an fp32 result: the only partial matrix is the result, written in place
-    const bool direct = splits == 1 && a.K > 0 && out32 && !out16;
-    if (direct) a.partial = out32;
     // the packed codes go through the pipelined kernel for 1/2/4 bits with DMA-aligned arrays
     // (codes 16-byte, scale/min 4-byte aligned); 8-bit codes through the register-decoding kernel
     const bool v2_packed = mode == DW_B_PACKED && (a.bits == 1 || a.bits == 2 || a.bits == 4) &&
@@ -834,7 +855,21 @@ int launch_dw_gemm(DwArgs a, int mode, bool with_db, float* out32, uint16_t* out
     // resource's 31-bit range)
     const bool v2_ragged = mode == DW_B_BF16 && a.ldd < ((int64_t)1 << 24) && a.ldx < ((int64_t)1 << 24) &&
                            a.N < ((int64_t)1 << 20);
-    if ((mode == DW_B_BF16 || v2_packed) && (ragged ? v2_ragged : v2_offsets) && a.K > 0) {
+    const bool v2 = (mode == DW_B_BF16 || v2_packed) && (ragged ? v2_ragged : v2_offsets) && a.K > 0;
+    // One split: the only partial matrix is the result. An fp32 one is written in place (and rounded by the reduce if
+    // it is wanted in bf16 too); a bf16 one alone by the O16 instances, whose row offsets need N as the ragged ones do.
+    const bool one = splits == 1 && a.K > 0;
+    const bool o16 = one && v2 && mode == DW_B_BF16 && !out32 && a.N < ((int64_t)1 << 20);
+    const bool direct = one && (out32 || o16);
+    if (direct) a.partial = out32;
+    a.out16 = out16;
+    const auto reduce = [&](int used) {
+        if (!direct)
+            launch_dw_reduce(a.partial, used, a.M * a.N, out32, out16, a.db_partial, a.M, with_db ? db : nullptr, st);
+        else if (out32 && out16)
+            launch_dw_reduce(out32, used, a.M * a.N, nullptr, out16, nullptr, a.M, nullptr, st);
+    };
+    if (v2) {
         // the transpose-free kernel: 32-token tiles, split at the same token boundaries as the
         // 64-token kernel, so both accumulate the same 16-token MFMA steps in the same order
         // (K % 32 == 0 and N % 256 == 0 make the group count K N / g even, so the scale/min dword
@@ -849,32 +884,36 @@ int launch_dw_gemm(DwArgs a, int mode, bool with_db, float* out32, uint16_t* out
         const int bnt = dw_tile_cols(a.M, a.N);
         const int64_t W = ((a.M + bmt - 1) / bmt) * ((a.N + bnt - 1) / bnt) * used;
         const dim3 grid((unsigned)(DW_XCDS * ((W + DW_XCDS - 1) / DW_XCDS)));
-#define DOPT_DW2T(BITS_, BMT_)                                                                                     \
-    do {                                                                                                           \
-        if (with_db) hipLaunchKernelGGL((dw_gemm_v2_kernel<BITS_, true, 4, BMT_>), grid, dim3(256), 0, st, a);      \
-        else hipLaunchKernelGGL((dw_gemm_v2_kernel<BITS_, false, 4, BMT_>), grid, dim3(256), 0, st, a);             \
-    } while (0)
-#define DOPT_DW2(BITS_)                          \
-    do {                                         \
-        if (bmt == 128) DOPT_DW2T(BITS_, 128);   \
-        else DOPT_DW2T(BITS_, 256);              \
-    } while (0)
-#define DOPT_DW2R(BMT_, BNT_)                                                                                          \
+#define DOPT_DW2T(BITS_, BMT_, BNT_, RAG_, O16_)                                                                      \
     do {                                                                                                               \
-        if (with_db) hipLaunchKernelGGL((dw_gemm_v2_kernel<0, true, 4, BMT_, BNT_, true>), grid, dim3(256), 0, st, a);  \
-        else hipLaunchKernelGGL((dw_gemm_v2_kernel<0, false, 4, BMT_, BNT_, true>), grid, dim3(256), 0, st, a);         \
+        if (with_db)                                                                                                   \
+            hipLaunchKernelGGL((dw_gemm_v2_kernel<BITS_, true, 4, BMT_, BNT_, RAG_, O16_>), grid, dim3(256), 0, st, a); \
+        else                                                                                                           \
+            hipLaunchKernelGGL((dw_gemm_v2_kernel<BITS_, false, 4, BMT_, BNT_, RAG_, O16_>), grid, dim3(256), 0, st, a); \
     } while (0)
-        if (ragged && bmt == 256) DOPT_DW2R(256, 256);
-        else if (ragged && bnt == 256) DOPT_DW2R(128, 256);
-        else if (ragged) DOPT_DW2R(128, 128);
-        else if (mode == DW_B_BF16) DOPT_DW2(0);
+#define DOPT_DW2(BITS_)                                          \
+    do {                                                         \
+        if (bmt == 128) DOPT_DW2T(BITS_, 128, 256, false, false); \
+        else DOPT_DW2T(BITS_, 256, 256, false, false);            \
+    } while (0)
+// bf16 x_hat: whole and ragged tiles, fp32 partials or the bf16 result
+#define DOPT_DW2B(O16_)                                                 \
+    do {                                                                \
+        if (ragged && bmt == 256) DOPT_DW2T(0, 256, 256, true, O16_);    \
+        else if (ragged && bnt == 256) DOPT_DW2T(0, 128, 256, true, O16_); \
+        else if (ragged) DOPT_DW2T(0, 128, 128, true, O16_);             \
+        else if (bmt == 128) DOPT_DW2T(0, 128, 256, false, O16_);        \
+        else DOPT_DW2T(0, 256, 256, false, O16_);                        \
+    } while (0)
+        if (mode == DW_B_BF16 && o16) DOPT_DW2B(true);
+        else if (mode == DW_B_BF16) DOPT_DW2B(false);
         else if (a.bits == 1) DOPT_DW2(1);
         else if (a.bits == 2) DOPT_DW2(2);
         else DOPT_DW2(4);
-#undef DOPT_DW2R
+#undef DOPT_DW2B
 #undef DOPT_DW2
 #undef DOPT_DW2T
-        if (!direct) launch_dw_reduce(a.partial, used, a.M * a.N, out32, out16, a.db_partial, a.M, with_db ? db : nullptr, st);
+        reduce(used);
         return 0;
     }
     if (a.M % BM != 0 || a.N % BN != 0) {
@@ -903,7 +942,7 @@ int launch_dw_gemm(DwArgs a, int mode, bool with_db, float* out32, uint16_t* out
 #undef DOPT_DW_DB
 #undef DOPT_DW
     }
-    if (!direct) launch_dw_reduce(a.partial, used, a.M * a.N, out32, out16, a.db_partial, a.M, with_db ? db : nullptr, st);
+    reduce(used);
     return 0;
 }
 

@@ -86,9 +86,9 @@ def dw_any_preferred(M: int, N: int, K: int, bias_grad: bool) -> bool:
     """Whether a Linear layer's weight gradient goes through dw_gemm_any: always when both feature counts are
     multiples of 256 (there it runs dw_gemm's kernels with the same result, through a native operator that costs
     the host about half of dw_gemm's Python one). For other multiples of 8 it takes the place of torch's product
-    (and sum): with a bias gradient it was the faster one on every shape measured (8 x 8 to 3008 x 3072 over 12 to
-    25216 tokens, 1.05x to 5x); without one torch's product alone is faster over few tokens (1024 x 1024 over 333:
-    8 us against 14)."""
+    (and sum): with a bias gradient it was the faster one on every shape measured, for fp32 and bf16 weights
+    (8 x 8 to 8200 x 8200 over 11 to 30000 tokens, 1.05x to 6x); without one torch's product alone is faster over few
+    tokens (1024 x 1024 over 333: 8 us against 14)."""
     if M <= 0 or N <= 0 or M % 8 or N % 8 or max(M, N) >= 1 << 20:
         return False
     return bias_grad or K >= 1024 or dw_gemm_supported(M, N)

@@ -69,6 +69,18 @@ def test_packed_operand_equals_dequantized(bits, g, K, M, N):
     check_close(got, dy, x_hat)
 
 
+@pytest.mark.parametrize("K", [64, 45, 2048])
+@pytest.mark.parametrize("bits", [1, 2, 4, 8])
+def test_packed_bf16_result(bits, K):
+    """From codes too, the bf16 result is the fp32 one rounded (one split over few tokens, several over many)."""
+    M, N, g = 1024, 1024, 256
+    dy, x = operands(K, M, N, bits)
+    packed, scale, xmin = ops.quant_pack_triton(x.reshape(1, -1, g), bits, g, False, 0, True, 3.0)
+    want, wdb = ops.dw_gemm(dy, None, packed, scale, xmin, N, bits, g, True, torch.float32)
+    got, gdb = ops.dw_gemm(dy, None, packed, scale, xmin, N, bits, g, True, torch.bfloat16)
+    assert torch.equal(got, want.to(torch.bfloat16)) and torch.equal(gdb, wdb)
+
+
 def test_no_tokens_and_errors():
     dy = torch.empty((0, 256), device=DEV, dtype=torch.bfloat16)
     x = torch.empty((0, 256), device=DEV, dtype=torch.bfloat16)

@@ -55,6 +55,37 @@ def test_ragged_shapes(M, N, K, pad):
         assert bool((db[M if with_db else 0:] == 7).all())
 
 
+# one split (the last two: several), whole and ragged tiles of every shape
+@pytest.mark.parametrize("M,N,K", [(8, 8, 1), (136, 248, 20), (264, 136, 40), (1288, 1544, 97), (2056, 2104, 65),
+                                   (4096, 4096, 64), (1024, 768, 32), (384, 192, 999), (768, 768, 985)])
+def test_bf16_result(M, N, K):
+    """The bf16 result is the fp32 one rounded, asked for alone or beside it; with one split it is written at once
+    and the workspace stays as it was."""
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    dy = torch.randn((K, M), generator=g, device=DEV).to(torch.bfloat16)
+    x = torch.randn((K, N), generator=g, device=DEV).to(torch.bfloat16)
+    L = _lib.lib()
+    n = max(L.dopt_dw_gemm_any_workspace_floats(M, N, K), 4)
+    got = {}
+    for f32, b16 in ((True, False), (False, True), (True, True)):
+        ws = torch.full((n,), 7.0, device=DEV)
+        out32 = torch.full((M * N + 8,), 7.0, device=DEV)
+        out16 = torch.full((M * N + 8,), 7.0, device=DEV, dtype=torch.bfloat16)
+        db = torch.full((M + 8,), 7.0, device=DEV)
+        rc = L.dopt_dw_gemm_any(dy.data_ptr(), M, x.data_ptr(), N, M, N, K, ws.data_ptr(), out32.data_ptr() if f32 else None,
+                                out16.data_ptr() if b16 else None, db.data_ptr(), torch.cuda.current_stream().cuda_stream)
+        _lib.check(rc, "dw_gemm_any")
+        got[f32, b16] = out32, out16, db
+        assert bool((out32[M * N if f32 else 0:] == 7).all()) and bool((out16[M * N if b16 else 0:] == 7).all())
+        assert bool((db[M:] == 7).all()) and torch.equal(db, got[True, False][2])
+        if K <= 97:
+            assert bool((ws == 7).all())
+    want = got[True, False][0][:M * N]
+    assert torch.equal(got[True, True][0][:M * N], want)
+    for key in ((False, True), (True, True)):
+        assert torch.equal(got[key][1][:M * N], want.to(torch.bfloat16))
+
+
 @pytest.mark.parametrize("M,N,K", [(256, 256, 777), (512, 768, 2048), (768, 768, 985), (1024, 1280, 333), (256, 512, 64)])
 def test_equals_dw_gemm(M, N, K):
     g = torch.Generator(device=DEV).manual_seed(K)
