@@ -1047,7 +1047,7 @@ static bool dw_any_shape(int64_t M, int64_t N, int64_t K) {
 }
 
 int64_t dopt_dw_gemm_any_workspace_floats(int64_t M, int64_t N, int64_t K) {
-    return dw_any_shape(M, N, K) ? dopt::dw_workspace_floats(M, N, K) : 0;
+    return dw_any_shape(M, N, K) ? dopt::dw_any_workspace_floats(M, N, K) : 0;
 }
 
 int dopt_dw_gemm_any(const void* dy, int64_t ldd, const void* x_hat, int64_t ldx, int64_t M, int64_t N, int64_t K,

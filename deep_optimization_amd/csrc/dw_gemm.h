@@ -29,6 +29,7 @@ struct DwArgs {
 
 int dw_splits(int64_t M, int64_t N, int64_t K);
 int64_t dw_workspace_floats(int64_t M, int64_t N, int64_t K);
+int64_t dw_any_workspace_floats(int64_t M, int64_t N, int64_t K);
 int launch_dw_gemm(DwArgs a, int mode, bool with_db, float* out32, uint16_t* out16, float* db, hipStream_t st);
 
 }  // namespace dopt

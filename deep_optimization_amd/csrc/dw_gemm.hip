@@ -840,6 +840,11 @@ int64_t dw_workspace_floats(int64_t M, int64_t N, int64_t K) {
     return (int64_t)s * M * N + (int64_t)s * M;
 }
 
+// bf16 x_hat within the ragged instances' offsets: one split writes the result and uses none (launch_dw_gemm)
+int64_t dw_any_workspace_floats(int64_t M, int64_t N, int64_t K) {
+    return dw_splits(M, N, K) == 1 ? 0 : dw_workspace_floats(M, N, K);
+}
+
 int launch_dw_gemm(DwArgs a, int mode, bool with_db, float* out32, uint16_t* out16, float* db, hipStream_t st) {
     const int splits = dw_splits(a.M, a.N, a.K);
     // the packed codes go through the pipelined kernel for 1/2/4 bits with DMA-aligned arrays

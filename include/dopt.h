@@ -423,7 +423,8 @@ int dopt_dw_gemm(const void* dy, int64_t ldd, const void* x_hat, int64_t ldx, co
 /* No counterpart in the reference. dopt_dw_gemm with bf16 x_hat for any K and any M, N that are multiples of 8
  * (below 2^20): the Linear layers whose feature counts dopt_dw_gemm does not take. The same sums (and, where
  * dopt_dw_gemm takes the shape, the same results bit for bit); workspace of
- * dopt_dw_gemm_any_workspace_floats(M, N, K) floats; ldd, ldx multiples of 8, >= M, N and below 2^24. */
+ * dopt_dw_gemm_any_workspace_floats(M, N, K) floats (0 where K is not split and the result written at once; the
+ * pointer must not be null all the same); ldd, ldx multiples of 8, >= M, N and below 2^24. */
 int64_t dopt_dw_gemm_any_workspace_floats(int64_t M, int64_t N, int64_t K);
 int dopt_dw_gemm_any(const void* dy, int64_t ldd, const void* x_hat, int64_t ldx, int64_t M, int64_t N, int64_t K,
                      float* workspace, float* dw_f32, void* dw_bf16, float* db, void* stream);

@@ -71,6 +71,14 @@ class TestValidationWithoutDevice:
         for M, N, K in ((200, 200, 208), (109, 491, 80), (257, 827, 96)):
             assert L.dopt_fp8_gemm_kn_copy_preferred(M, N, K) == 1, (M, N, K)
 
+    def test_weight_gradient_workspace(self):
+        """Split partials only: an unsplit product (large outputs, few tokens) needs none."""
+        floats = _lib.lib().dopt_dw_gemm_any_workspace_floats
+        for M, N, K in ((8, 8, 1), (1000, 2048, 32), (3072, 3072, 333), (8200, 8200, 4096), (256, 256, 0)):
+            assert floats(M, N, K) == 0, (M, N, K)
+        for M, N, K in ((768, 768, 25216), (384, 192, 999)):
+            assert floats(M, N, K) >= 2 * (M * N + M), (M, N, K)
+
     def test_bad_bits_is_value_error(self):
         assert self.qp(bits=3) == _lib.EBITS
         with pytest.raises(ValueError, match="bits must be one of"):
