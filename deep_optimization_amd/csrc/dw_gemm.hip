@@ -823,6 +823,11 @@ int dw_tile_cols(int64_t M, int64_t N) {
 // batch 128: 7, 9 and 14 splits as before); with few tokens the partials had cost more than the product:
 // 1024 x 1024 over 333 tokens 24.0 -> 13.7 us (with the direct result below), 768 x 768 over 985 23.9 -> 15.7,
 // 3072 x 3072 over 4001 185 -> 105.
+// The terms are a bf16 x_hat's, the layers' default. The kernels that decode codes take longer per slab and would want
+// more splits: from 8-bit codes, or over a token count that is no multiple of 32, some shapes run 5 to 18% slower than
+// with the first limit alone (768 x 3072 over 985 tokens 42 -> 49 us; 768 x 768 over 4096 from 8-bit codes 46 -> 63).
+// A fifth more splits for every kernel had gained them little and cost a bf16 x_hat up to 9% (768 x 2304 over 8192
+// 50.2 -> 54.3).
 int dw_splits(int64_t M, int64_t N, int64_t K) {
     const int bmt = dw_tile_rows(M, N), bnt = dw_tile_cols(M, N);
     const int64_t tiles = std::max<int64_t>(((M + bmt - 1) / bmt) * ((N + bnt - 1) / bnt), 1);
