@@ -77,9 +77,14 @@ static int qp_rn(const QuantPackArgs& a, int rn, int pre, hipStream_t s) {
             case RN_NEAREST:
                 // threshold codes on the bf16 grid where the squash applies (4 and 8 bits would need 15 and
                 // 255 thresholds; an fp32 or fp16 input has no grid on which the evaluated squash was shown
-                // non-decreasing); a negative or NaN alpha keeps the per-element clamp's own arithmetic
+                // non-decreasing); a negative or NaN alpha keeps the per-element clamp's own arithmetic.
+                // Up to 2^20 elements at 2 bits and groups of 256 and more keep the per-element form: too few waves to
+                // fill the CUs, so a lane's chain of instructions is the time, and its thresholds are the longer
+                // one (g = 256, us, per element / thresholds: 2^16 elements 3.54 / 3.92, 2^20 3.71 / 4.02, 3 * 2^19
+                // 4.30 / 4.05, 2^23 8.64 / 5.52; at 1 bit or g <= 128 the thresholds are no slower at any size)
                 if constexpr (DT == DT_BF16 && BITS <= 2) {
-                    if ((a.flags & FL_SQUASH) && (!(a.flags & FL_CLAMP) || a.clamp_alpha >= 0.0f))
+                    const bool few = BITS == 2 && G >= 256 && (uint64_t)a.n_groups * G <= (1u << 20);
+                    if (!few && (a.flags & FL_SQUASH) && (!(a.flags & FL_CLAMP) || a.clamp_alpha >= 0.0f))
                         return qp_launch<DT, BITS, G, RN_NEAREST, PRE_SQ16>(a, s);
                 }
                 return qp_launch<DT, BITS, G, RN_NEAREST, PRE_REF>(a, s);

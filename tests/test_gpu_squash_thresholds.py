@@ -78,3 +78,19 @@ def test_tiles_and_small_counts(bits, g, hw, n):
     args = (bits, g, True, 3.0, True, 0, None, 0, 0, torch.float32)
     for got, want in zip(ops.quant_pack_tiles(x, *args), ops.quant_pack_tiles(x.float(), *args)):
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("g,hw,n", [(256, (16, 48), 461), (1024, (32, 64), 175)])
+def test_tiles_of_many_groups(g, hw, n):
+    """2 bits and groups of 256 and more take the thresholds above 2^20 elements only: the tile layout there, with a
+    partial wave, and flat groups on both sides of the line."""
+    gen = torch.Generator(device=DEV).manual_seed(n)
+    args = (2, g, True, 3.0, True, 0, None, 0, 0, torch.float32)
+    x = torch.randn((n, 3, *hw), generator=gen, device=DEV).to(torch.bfloat16)
+    assert x.numel() > 1 << 20
+    for got, want in zip(ops.quant_pack_tiles(x, *args), ops.quant_pack_tiles(x.float(), *args)):
+        assert torch.equal(got, want)
+    for groups in ((1 << 20) // g - 1, (1 << 20) // g, (1 << 20) // g + 1):
+        x = torch.randn((1, groups, g), generator=gen, device=DEV).to(torch.bfloat16)
+        for got, want in zip(ops.quant_pack(x, *args), ops.quant_pack(x.float(), *args)):
+            assert torch.equal(got, want)
