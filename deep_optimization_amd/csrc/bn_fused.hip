@@ -778,7 +778,7 @@ __global__ __launch_bounds__(TPB) void bn_fwd_kernel(BnFwdArgs a, int lg, int bi
 // then the same blocks normalized and quantized, so x is read once and no second kernel starts. One kernel's start
 // and drain are most of such a layer's time. Up to two chunks: 64 elements a lane in registers. bf16, statistics and
 // forward -> whole, us: [64, 512, 7, 7] with ReLU 15.0 -> 8.2, [128, 2048, 7, 7] 35.0 -> 24.1, [64, 1024, 14, 14] with
-// ReLU (two chunks) 28.1 -> 22.3; 64 workgroups of two chunks ([64, 64, 14, 14]) no slower.
+// ReLU (two chunks) 28.1 -> 22.3; [64, 64, 14, 14] (two chunks) 12.3 -> 11.9.
 template <int DT, int MODE, int V, bool R6, bool THR, int CH>
 __global__ __launch_bounds__(TPB) void bn_fwd_whole_kernel(BnFwdArgs a, int lg, int bits) {
     const int64_t c = channel_of<V>();
@@ -1150,8 +1150,12 @@ void bwd_whole(const BnBwdArgs& a, int mode, int group, int bits, hipStream_t s)
 }
 
 // Channels of at most this many chunks take the whole-channel kernels (quantized modes without ALAM, and every
-// access width but the element and two-element ones of rows below 8 elements).
-constexpr int64_t WHOLE_CHUNKS = 2;
+// access width but the element and two-element ones of rows below 8 elements). In the forward few channels whose
+// second chunk is full (all 64 elements of a lane) are the exception at widths 8 and 4: a workgroup per channel
+// is half the workgroups of the two kernels and twice the serial work, 0.2 to 0.8 us more than a second launch
+// costs (bf16, us, two kernels / whole: [64, 4, 16, 16] with ReLU 9.6 / 10.2, [16, 64, 32, 32] 10.2 / 10.6; equal at 192
+// channels, and with one block of 2048 elements less the whole kernel is never slower).
+constexpr int64_t WHOLE_CHUNKS = 2, WHOLE_FWD_ELEMS = (2 * ITER - 1) * WG_ELEMS, WHOLE_FWD_CHANNELS = 128;
 
 bool whole_channel(int64_t nchunks, int mode, int vw) {
     return mode != BN_NORM && nchunks <= WHOLE_CHUNKS && (vw == 8 || vw == 4 || vw == 0);
@@ -1169,6 +1173,7 @@ bool whole_channel(int64_t nchunks, int mode, int vw) {
 
 bool launch_bn_fwd_whole(const BnFwdArgs& a, int dt, int mode, int group, int bits, int vw, hipStream_t s) {
     if (!whole_channel(a.nchunks, mode, vw)) return false;
+    if (vw != 0 && a.g.N * a.g.HW > WHOLE_FWD_ELEMS && a.g.C <= WHOLE_FWD_CHANNELS) return false;
     switch (dt) {
         case DT_F32: DOPT_BN_WHOLE(fwd_whole, DT_F32, a, mode, group, bits, s); break;
         case DT_F16: DOPT_BN_WHOLE(fwd_whole, DT_F16, a, mode, group, bits, s); break;

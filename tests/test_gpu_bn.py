@@ -617,9 +617,10 @@ def test_short_and_unaligned_rows(N, C, HW, dtype, kind, bits, shift):
 
 
 # channels of one and two 8192-element chunks (the whole-channel kernels) at the edges of the chunks and of the lanes'
-# blocks, and one element group beyond them (the kernel pairs), in each access width
+# blocks, and one element group beyond them (the kernel pairs), in each access width; two full chunks at widths 8 and 4
+# with few channels (the forward's kernel pair) and with more (the whole-channel kernel)
 CHANNELS = [(1, 3, 32), (1, 3, 8192), (1, 3, 8192 + 32), (1, 3, 16384), (1, 3, 16384 + 32), (2, 8, 4096 - 16), (8, 2, 4 * 257),
-            (96, 16, 49), (160, 8, 51), (224, 5, 49), (352, 3, 49)]
+            (96, 16, 49), (160, 8, 51), (224, 5, 49), (352, 3, 49), (1, 136, 16384)]
 
 
 @pytest.mark.parametrize("N,C,HW", CHANNELS)
