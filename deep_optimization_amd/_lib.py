@@ -32,6 +32,7 @@ EXPORTS = (
     "dopt_fp8_gemm_kn",
     "dopt_fp8_gemm_kn_preferred",
     "dopt_fp8_gemm_kn_copy_preferred",
+    "dopt_fp8_gemm_tile",
     "dopt_fp8_pack_kmajor",
     "dopt_fp8_pack_kmajor_padded",
     "dopt_relu_pack",
@@ -105,6 +106,8 @@ def lib() -> ctypes.CDLL:
         L.dopt_fp8_gemm_kn_preferred.restype = i32
         L.dopt_fp8_gemm_kn_copy_preferred.argtypes = [i64, i64, i64]
         L.dopt_fp8_gemm_kn_copy_preferred.restype = i32
+        L.dopt_fp8_gemm_tile.argtypes = [i64, i64, i64, i32]
+        L.dopt_fp8_gemm_tile.restype = i32
         L.dopt_fp8_pack_kmajor.argtypes = [vp, i64, i64, i64, i64, vp, i64, vp]
         L.dopt_fp8_pack_kmajor.restype = i32
         L.dopt_fp8_pack_kmajor_padded.argtypes = [vp, i64, i64, i64, i64, vp, i64, i64, vp]

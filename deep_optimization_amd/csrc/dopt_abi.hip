@@ -20,6 +20,7 @@ int launch_fp8_gemm_nt(const uint8_t* A, const uint8_t* B, int64_t M, int64_t N,
 int launch_fp8_gemm_kn(const uint8_t* A, const uint8_t* B, int64_t M, int64_t N, int64_t K, int64_t b_rows, int64_t lda,
                        int64_t ldb, float out_scale, uint16_t* C, int64_t ldc, hipStream_t s);
 bool fp8_gemm_kn_preferred(int64_t M, int64_t N, int64_t K, bool copied);
+int fp8_gemm_tile(int64_t M, int64_t N, int64_t K, bool kn);
 int launch_fp8_pack(const uint8_t* src, int64_t rows, int64_t cols, int64_t stride_r, int64_t stride_c, uint8_t* dst,
                     int64_t ld_dst, int64_t cols_out, hipStream_t s);
 int launch_relu_pack(const void* x, int dt, void* y, uint32_t* packed, uint64_t n, int bits, bool relu6, hipStream_t s);
@@ -448,6 +449,11 @@ static int fp8_kn_preferred(int64_t M, int64_t N, int64_t K, bool copied) {
 int dopt_fp8_gemm_kn_preferred(int64_t M, int64_t N, int64_t K) { return fp8_kn_preferred(M, N, K, false); }
 
 int dopt_fp8_gemm_kn_copy_preferred(int64_t M, int64_t N, int64_t K) { return fp8_kn_preferred(M, N, K, true); }
+
+int dopt_fp8_gemm_tile(int64_t M, int64_t N, int64_t K, int kn) {
+    if (M <= 0 || N <= 0 || K < 0) return fail(DOPT_EINVAL, "fp8_gemm_tile: M and N must be positive and K not negative");
+    return dopt::fp8_gemm_tile(M, N, K, kn != 0);
+}
 
 int dopt_fp8_gemm_kn(const uint8_t* A, const uint8_t* B, int64_t M, int64_t N, int64_t K, int64_t b_rows, int64_t lda,
                      int64_t ldb, float out_scale, void* C, int64_t ldc, void* stream) {

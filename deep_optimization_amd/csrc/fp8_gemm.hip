@@ -115,6 +115,12 @@ int launch_fp8_gemm_kn(const uint8_t* A, const uint8_t* B, int64_t M, int64_t N,
     return fp8_gemm_mid_launch<128, 128, true>(p, s);
 }
 
+// the index in TILE_COST of the tile a product gets
+int fp8_gemm_tile(int64_t M, int64_t N, int64_t K, bool kn) {
+    float us;
+    return plan(M, N, K, device_cu_count(), kn, &us);
+}
+
 // Whether reading B as it lies is estimated to be faster than packing it (a launch of about 3 us and its
 // bytes) for launch_fp8_gemm_nt. Both ways timed on 16 shapes from 1 x 4096 x 4096 to 8192^3; us, packed ->
 // as it lies: 985 x 768 x 1536 8.5 -> 5.5, 64 x 4096 x 4096 17.1 -> 6.7, 1024^3 7.8 -> 4.8, 2048^3

@@ -1,5 +1,5 @@
-// FP8 (OCP e4m3) scaled GEMM for outputs too small to give every CU a 128 x 128 or 256 x 256 tile
-// (fp8_gemm.h): a workgroup computes a (16 MT) x (16 NT) tile and its NW waves split K between them.
+// FP8 (OCP e4m3) scaled GEMM of at most 16 rows (larger ones: fp8_gemm_mid.h, fp8_gemm.h): a workgroup computes a
+// (16 MT) x (16 NT) tile and its NW waves split K between them; the launcher uses 16 x 16 tiles and 8 waves.
 // Same operands, result and edge handling: C[m][n] = bf16(out_scale * sum_k A[m][k] * B[n][k]), fp32
 // sums, one rounding; any M, N; K a multiple of 16.
 //
@@ -54,8 +54,8 @@ __global__ __launch_bounds__(64 * NW) void fp8_gemm_small_kernel(Fp8GemmArgs p) 
     struct Frags {
         v8i_t a[MT], b[NT];
     };
-    // (the K offset is at most 2^23 and the row offsets at most 64 * 2^23: a lane past its rows stays
-    // beyond the range)
+    // (the K offset is at most 2^23 and the row offsets at most 16 * 2^23 for the 16 x 16 tile: a lane past its rows
+    // stays beyond the range)
     auto load = [&](__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t k0, uint32_t past0, uint32_t past1)
                     __attribute__((always_inline)) {
         const v4u_t x0 = __builtin_amdgcn_raw_buffer_load_b128(r, off | past0, (int)k0, 0);

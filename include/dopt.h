@@ -176,6 +176,13 @@ int dopt_fp8_gemm_kn_preferred(int64_t M, int64_t N, int64_t K);
 int dopt_fp8_gemm_kn_copy_preferred(int64_t M, int64_t N, int64_t K);
 
 /*
+ * The workgroup tile that dopt_fp8_gemm_nt (kn = 0) or dopt_fp8_gemm_kn (kn = 1) takes for a product on the current
+ * device: 0 16 x 16, 1 32 x 64, 2 64 x 64, 3 128 x 64, 4 128 x 128, 5 128 x 128 with two workgroups per CU,
+ * 6 256 x 256 (kn: 1 to 4). Negative: an error code.
+ */
+int dopt_fp8_gemm_tile(int64_t M, int64_t N, int64_t K, int kn);
+
+/*
  * Layout conversion for dopt_fp8_gemm_nt: dst[r * ld_dst + c] = src[r * stride_r + c * stride_c]
  * (byte matrices, element strides in bytes). The reference's Triton_Linear
  * (Activation_Compression/triton_kernel/linear.py:43-95) takes A [M, K] and B [K, N] with arbitrary

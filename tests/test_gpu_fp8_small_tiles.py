@@ -19,11 +19,18 @@ DEV = "cuda"
 NAN8 = 0x7F  # an e4m3 NaN encoding
 
 # (M, N) around 16, 32, 64 and 128; K around the 128-byte chunk, the four LDS stages and 8 waves' chunks;
-# and one shape per tile the launcher knows (the last four: 128 x 128 twice, 256 x 256 edge instances)
+# and at least one shape per tile the launcher knows (test_shapes_reach_every_tile); of the 256 x 256 edge instances the
+# persistent ones of either matrix instruction (an even slab count; 16x16x128 from K = 8192) and the other (an odd one)
 SHAPES = [(1, 1, 16), (16, 16, 128), (17, 15, 112), (1, 8, 2048), (15, 4097, 1040), (16, 700, 1152),
           (31, 65, 144), (32, 64, 512), (33, 63, 640), (64, 128, 384), (65, 129, 496), (63, 1000, 128),
           (300, 515, 272), (512, 512, 1024), (129, 4096, 1168), (1000, 1024, 2064), (257, 8193, 400),
-          (985, 3072, 768), (1030, 2100, 1296), (2050, 4100, 656), (4000, 4111, 1200), (3900, 4111, 8336)]
+          (985, 3072, 768), (1030, 2100, 1296), (2050, 4100, 656), (4000, 4111, 1200), (3900, 4111, 8336),
+          (520, 2001, 1008), (4090, 4090, 1296), (4090, 4090, 8336)]
+
+# ... and of a row-major B
+ROW_MAJOR_SHAPES = [(1, 16, 1), (17, 48, 100), (33, 64, 128), (64, 80, 513), (129, 144, 640), (985, 768, 1536),
+                    (300, 1040, 1111), (1000, 2064, 400), (2050, 3088, 272), (70, 33, 65), (262, 3804, 187),
+                    (1000, 777, 1001), (300, 5008, 3000), (520, 2001, 1000)]
 
 
 def fp8(shape, gen):
@@ -38,11 +45,21 @@ def check(c, a, b, scale):
     assert bool((err <= 2 ** -8 * ref.abs() + 2 ** -12 * mag).all()), float((err - 2 ** -8 * ref.abs()).max())
 
 
+def test_shapes_reach_every_tile():
+    tile = _lib.lib().dopt_fp8_gemm_tile
+    assert {tile(*s, 0) for s in SHAPES} == set(range(7))
+    # the 256 x 256 tile's three edge instances: (slab count even, K >= 8192)
+    slabs = {((K + 127) // 128 % 2 == 0, K >= 8192) for M, N, K in SHAPES if tile(M, N, K, 0) == 6}
+    assert {(True, True), (True, False), (False, False)} <= slabs
+    assert {tile(M, N, (K + 15) // 16 * 16, 1) for M, N, K in ROW_MAJOR_SHAPES} == {1, 2, 3, 4}
+    assert tile(0, 16, 16, 0) == _lib.EINVAL and tile(16, 16, -1, 1) == _lib.EINVAL
+
+
 @pytest.mark.parametrize("M,N,K", SHAPES)
 @pytest.mark.parametrize("padded", [False, True])
 def test_tile_edges(M, N, K, padded):
-    """Contiguous operands (16-byte stores where N % 8 == 0), and padded rows whose padding holds NaN with an
-    odd ldc (element stores) and a sentinel around C."""
+    """Contiguous operands, and padded rows whose padding holds NaN with an odd ldc (unaligned 16-byte stores, element
+    stores for the last chunk) and a sentinel around C."""
     gen = torch.Generator(device=DEV).manual_seed(M + 3 * N + K)
     lda, ldb, ldc = (K + 16, K + 48, N + 5) if padded else (K, K, N)
     a, b = fp8((M, lda), gen), fp8((N, ldb), gen)
@@ -61,9 +78,7 @@ def test_tile_edges(M, N, K, padded):
     assert torch.equal(c, first)  # the split K is summed in a fixed order
 
 
-@pytest.mark.parametrize("M,N,K", [(1, 16, 1), (17, 48, 100), (33, 64, 128), (64, 80, 513), (129, 144, 640), (985, 768, 1536),
-                                   (300, 1040, 1111), (1000, 2064, 400), (2050, 3088, 272), (70, 33, 65), (262, 3804, 187),
-                                   (1000, 777, 1001)])
+@pytest.mark.parametrize("M,N,K", ROW_MAJOR_SHAPES)
 @pytest.mark.parametrize("padded", [False, True])
 def test_row_major_b(M, N, K, padded):
     """B in [K, N] rows, at the edges of every tile and of the slabs, with 0 to 15 rows less than A's padded K and

@@ -584,9 +584,9 @@ def test_fp8_gemm_parity(M, N, K):
                                    (4095, 4097, 4112), (300, 200, 0), (257, 255, 8336), (600, 520, 8448)])
 def test_fp8_gemm_ragged_shapes(M, N, K):
     """Edge tiles (M, N not multiples of 256, K a multiple of 16 but not of 64; K = 0 gives zeros),
-    through the C ABI with padded row strides: lda, ldb > K, ldc > N (odd, so element stores), and a
-    sentinel around the M x N block of C that must stay untouched. K = 8336 and 8448 (an even slab
-    count from K = 8192) take the 16x16x128 persistent kernel's edge instance."""
+    through the C ABI with padded row strides: lda, ldb > K, ldc > N (odd, so unaligned 16-byte stores and element
+    stores for the last chunk), and a sentinel around the M x N block of C that must stay untouched. (The kernel
+    each tile shape gets is covered in test_gpu_fp8_small_tiles.py.)"""
     gen = torch.Generator(device=DEV).manual_seed(M * 7 + N + K)
     lda, ldb, ldc = K + 32, K + 48, N + 3
     a_buf = torch.randn(M, lda, generator=gen, device=DEV)
@@ -615,7 +615,7 @@ def test_fp8_gemm_ragged_shapes(M, N, K):
 
 
 def test_fp8_gemm_operator_odd_n():
-    """act_lib::fp8_gemm_nt with N % 8 != 0 (ldc = N: element stores) equals the fp32 matmul."""
+    """act_lib::fp8_gemm_nt with N % 8 != 0 (ldc = N: unaligned stores) equals the fp32 matmul."""
     gen = torch.Generator(device=DEV).manual_seed(3)
     a8, sa = fp8_quantize(torch.randn(130, 96, generator=gen, device=DEV))
     b8, sb = fp8_quantize(torch.randn(67, 96, generator=gen, device=DEV))
