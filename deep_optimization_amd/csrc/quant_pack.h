@@ -203,8 +203,8 @@ __device__ __forceinline__ uint32_t swap_fields(uint32_t x, int d, uint32_t m) {
 // VALU instructions per element, two of them transcendental: on the ViT MLP activation (bf16
 // [128,197,3072], g = 512, 2-bit) the kernel was bound by them at 51.3 us (3.4 TB/s); it now takes 27.6 us
 // (6.3 TB/s; the nearest quantizer without the squash takes 25.3). Every part of it
-// is non-decreasing in x over the bf16 values (squash_half_tanh2 as evaluated here included: a test
-// walks all of them), so
+// is non-decreasing in x over the bf16 values and +-alpha (squash_half_tanh2 as evaluated here included: a test
+// walks all bf16 values and the fp32 values around them, where an alpha may lie), so
 //   - min and max of the squashed values are the squash of the values' min and max, which are packed
 //     16-bit integer min / max of the ordered bits;
 //   - code >= k exactly when x >= b_k, the smallest bf16 value whose code is >= k. A lane finds its b_k

@@ -30,6 +30,22 @@ def test_squash_is_non_decreasing_on_the_bf16_grid():
     assert bool((mn.flatten().diff() >= 0).all())
 
 
+def test_squash_is_non_decreasing_around_the_grid():
+    """... and over the clamp's alpha, which may lie between two grid values: the 16 fp32 values on either side of every
+    finite bf16 value, and runs of consecutive ones where the squash bends and saturates. (All fp32 values from -3.4e38
+    to 3.4e38 were checked once, 4.28e9 pairs of neighbours.)"""
+    grid = torch.arange(0, 0x7F80, device=DEV, dtype=torch.int32) << 16
+    near = (grid[:, None] + torch.arange(-16, 17, device=DEV, dtype=torch.int32)).flatten().clamp_min(0)
+    runs = [torch.arange(1 << 18, device=DEV, dtype=torch.int32) + torch.tensor(at, device=DEV).view(torch.int32)
+            for at in (1e-4, 0.099, 0.5, 2.69, 2.999, 4.0, 8.0)]
+    for bits in (near, *runs):
+        v = bits.view(torch.float32)
+        for x in (v, -v.flip(0)):
+            x = x.view(-1, 1, 1).expand(-1, 1, 64).contiguous()
+            _, _, mn = ops.quant_pack(x, 2, 64, False, 0.0, True, 0, None, 0, 0, torch.float32)
+            assert bool((mn.flatten().diff() >= 0).all())
+
+
 def cases(kind, n, g, gen):
     x = torch.randn((n, g), generator=gen, device=DEV)
     if kind == "relu":
@@ -94,3 +110,16 @@ def test_tiles_of_many_groups(g, hw, n):
         x = torch.randn((1, groups, g), generator=gen, device=DEV).to(torch.bfloat16)
         for got, want in zip(ops.quant_pack(x, *args), ops.quant_pack(x.float(), *args)):
             assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("alpha", [2.7, 3.0000002, 2.9999998, 0.1, 1e-3, 4.3, 1e-30, 100.1, INF])
+@pytest.mark.parametrize("bits", [1, 2])
+def test_alpha_between_grid_values(bits, alpha):
+    """An alpha that is no bf16 value, a few fp32 steps from one, tiny, in the saturation, or infinite."""
+    gen = torch.Generator(device=DEV).manual_seed(int(alpha * 1000) if alpha < INF else 1)
+    for kind in ("normal", "wide", "scales", "special"):
+        x = cases(kind, 4096 + 37, 256, gen).to(torch.bfloat16).view(1, -1, 256)
+        args = (bits, 256, True, alpha, True, 0, None, 0, 0, torch.float32)
+        for a, b in zip(ops.quant_pack(x, *args), ops.quant_pack(x.float(), *args)):
+            same = (a == b) | (a.isnan() & b.isnan()) if a.is_floating_point() else a == b
+            assert bool(same.all()), (kind, int((~same).sum()))
