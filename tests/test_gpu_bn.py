@@ -117,7 +117,9 @@ def check_stats(x, s, q):
     assert sums_close(npv(q), rq, mag2)
 
 
-SHAPES = [(4, 16, 16, 16), (8, 32, 14, 14), (16, 8, 7, 7), (32, 16, 28, 28), (8, 16, 5, 10)]
+# (the last four: rows below 8 elements, and rows of 8 and more in channels of no multiple of 8, an element or two an access)
+SHAPES = [(4, 16, 16, 16), (8, 32, 14, 14), (16, 8, 7, 7), (32, 16, 28, 28), (8, 16, 5, 10), (33, 4, 1, 5), (8, 4, 2, 3),
+          (3, 2, 3, 5), (9, 3, 2, 7)]
 DTYPES = [torch.bfloat16, torch.float32, torch.float16]
 
 
@@ -292,12 +294,12 @@ def test_errors():
 # ----------------------------------------------------------------------------- avg_alam
 # (shape, BLOCK_M, bits, alam_bits): run lengths dividing the group's code words (1: the plain
 # codes, noise in the reduce only; 16 and 64: runs spanning 2 and 8 lanes), every access width
-# (8 at 16x16 / 28x28, 4 at 14x14, 8 at any element at 5x10 and 7x7), groups of 32..256, and channels whose last
+# (8 at 16x16 / 28x28, 4 at 14x14, 8 at any element at 5x10 and 7x7, 1 at 1x5, 2 at 2x3), groups of 32..256, and channels whose last
 # wave of 512 elements lies partly past M (7x7: M = 1568); each in bf16, fp32 and fp16
 ACASES = [((4, 16, 16, 16), 64, 2, 2), ((4, 16, 16, 16), 64, 8, 8), ((16, 8, 14, 14), 128, 1, 2),
           ((16, 32, 14, 14), 128, 4, 4), ((32, 16, 28, 28), 512, 2, 16), ((32, 16, 28, 28), 512, 8, 64),
           ((32, 8, 7, 7), 64, 4, 4), ((32, 8, 5, 10), 64, 2, 1), ((32, 8, 5, 10), 64, 4, 2),
-          ((16, 16, 28, 28), 256, 1, 4)]
+          ((16, 16, 28, 28), 256, 1, 4), ((64, 8, 1, 5), 64, 2, 2), ((32, 8, 2, 3), 64, 4, 2)]
 
 
 @pytest.mark.parametrize("case", ACASES, ids=lambda c: "x".join(map(str, c[0])) + f"-B{c[1]}-b{c[2]}-A{c[3]}")
@@ -620,7 +622,8 @@ def test_short_and_unaligned_rows(N, C, HW, dtype, kind, bits, shift):
 # blocks, and one element group beyond them (the kernel pairs), in each access width; two full chunks at widths 8 and 4
 # with few channels (the forward's kernel pair) and with more (the whole-channel kernel)
 CHANNELS = [(1, 3, 32), (1, 3, 8192), (1, 3, 8192 + 32), (1, 3, 16384), (1, 3, 16384 + 32), (2, 8, 4096 - 16), (8, 2, 4 * 257),
-            (96, 16, 49), (160, 8, 51), (224, 5, 49), (352, 3, 49), (1, 136, 16384)]
+            (96, 16, 49), (160, 8, 51), (224, 5, 49), (352, 3, 49), (1, 136, 16384),
+            (32, 4, 36)]
 
 
 @pytest.mark.parametrize("N,C,HW", CHANNELS)

@@ -15,6 +15,7 @@ import pytest
 import torch
 
 import deep_optimization_amd  # noqa: F401
+from deep_optimization_amd import _lib
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -79,6 +80,25 @@ def test_packed_bf16_result(bits, K):
     want, wdb = ops.dw_gemm(dy, None, packed, scale, xmin, N, bits, g, True, torch.float32)
     got, gdb = ops.dw_gemm(dy, None, packed, scale, xmin, N, bits, g, True, torch.bfloat16)
     assert torch.equal(got, want.to(torch.bfloat16)) and torch.equal(gdb, wdb)
+
+
+@pytest.mark.parametrize("bias", [True, False])
+def test_rows_far_apart(bias):
+    """A row stride beyond the pipelined kernels' 32-bit offsets (2^24 elements over a ragged token count): the
+    register-staged kernel, bit for bit the others' result."""
+    K, M, N, ldd = 33, 256, 256, 1 << 24
+    dy, x = operands(K, M, N, 5)
+    wide = torch.empty((K, ldd), dtype=torch.bfloat16, device=DEV)
+    wide[:, :M] = dy
+    L = _lib.lib()
+    ws = torch.empty(max(L.dopt_dw_gemm_workspace_floats(M, N, K), 4), device=DEV)
+    dw, db = torch.empty((M, N), device=DEV), torch.empty(M, device=DEV)
+    rc = L.dopt_dw_gemm(wide.data_ptr(), ldd, x.data_ptr(), N, None, None, None, 0, 0, M, N, K, ws.data_ptr(), dw.data_ptr(),
+                        None, db.data_ptr() if bias else None, torch.cuda.current_stream().cuda_stream)
+    _lib.check(rc, "dw_gemm")
+    assert torch.equal(dw, ops.dw_gemm(dy, x, None, None, None, N, 0, 0, False, torch.float32)[0])
+    if bias:
+        assert bool(((db.double() - dy.double().sum(0)).abs() <= 1e-4 * dy.double().abs().sum(0) + 1e-6).all())
 
 
 def test_no_tokens_and_errors():

@@ -84,6 +84,7 @@ def test_bf16_result(M, N, K):
     assert torch.equal(got[True, True][0][:M * N], want)
     for key in ((False, True), (True, True)):
         assert torch.equal(got[key][1][:M * N], want.to(torch.bfloat16))
+    assert torch.equal(ops.dw_gemm_any(dy, x, False, torch.bfloat16)[0].view(-1), want.to(torch.bfloat16))  # without db
 
 
 @pytest.mark.parametrize("M,N,K", [(256, 256, 777), (512, 768, 2048), (768, 768, 985), (1024, 1280, 333), (256, 512, 64)])

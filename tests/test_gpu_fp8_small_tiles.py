@@ -20,12 +20,14 @@ NAN8 = 0x7F  # an e4m3 NaN encoding
 
 # (M, N) around 16, 32, 64 and 128; K around the 128-byte chunk, the four LDS stages and 8 waves' chunks;
 # and at least one shape per tile the launcher knows (test_shapes_reach_every_tile); of the 256 x 256 edge instances the
-# persistent ones of either matrix instruction (an even slab count; 16x16x128 from K = 8192) and the other (an odd one)
+# persistent ones of either matrix instruction (an even slab count; 16x16x128 from K = 8192) and the other (an odd one);
+# the last two: whole tiles of the two kernels that are not persistent
 SHAPES = [(1, 1, 16), (16, 16, 128), (17, 15, 112), (1, 8, 2048), (15, 4097, 1040), (16, 700, 1152),
           (31, 65, 144), (32, 64, 512), (33, 63, 640), (64, 128, 384), (65, 129, 496), (63, 1000, 128),
           (300, 515, 272), (512, 512, 1024), (129, 4096, 1168), (1000, 1024, 2064), (257, 8193, 400),
           (985, 3072, 768), (1030, 2100, 1296), (2050, 4100, 656), (4000, 4111, 1200), (3900, 4111, 8336),
-          (520, 2001, 1008), (4090, 4090, 1296), (4090, 4090, 8336)]
+          (520, 2001, 1008), (4090, 4090, 1296), (4090, 4090, 8336),
+          (1024, 3072, 256), (4096, 4096, 1152)]
 
 # ... and of a row-major B
 ROW_MAJOR_SHAPES = [(1, 16, 1), (17, 48, 100), (33, 64, 128), (64, 80, 513), (129, 144, 640), (985, 768, 1536),
